@@ -302,9 +302,9 @@ class Engine:
         self._check(lib().mjg_simulate(self.h, int(total_step), int(save_step)))
 
     def state(self):
-        x = np.zeros(3 * self.n); v = np.zeros(3 * self.n); f = np.zeros(3 * self.n)
+        x, v, f = (np.empty((self.n, 3)) for _ in range(3))
         self._check(lib().mjg_system_get_state(self.h, x.ctypes.data, v.ctypes.data, f.ctypes.data))
-        return x.reshape(-1, 3), v.reshape(-1, 3), f.reshape(-1, 3)
+        return x, v, f
 
 
 class Batch:
@@ -421,9 +421,9 @@ class Batch:
 
     def state(self, r: int):
         n = self.specs[r].n
-        x = np.zeros(3 * n); v = np.zeros(3 * n); f = np.zeros(3 * n)
+        x, v, f = (np.empty((n, 3)) for _ in range(3))
         self._check(lib().mjg_batch_get_state(self.h, r, x.ctypes.data, v.ctypes.data, f.ctypes.data))
-        return x.reshape(-1, 3), v.reshape(-1, 3), f.reshape(-1, 3)
+        return x, v, f
 
     def set_step_count(self, r: int, step: int):
         self._check(lib().mjg_batch_set_step_count(self.h, r, int(step)))

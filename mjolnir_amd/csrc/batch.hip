@@ -5,6 +5,7 @@
 // resident: each one owns a device arena sized by its footprint, and every launch runs the
 // replicas that are active, largest first, one workgroup each.
 #include "batch_kernels.hpp"
+#include "host_io.hpp"
 #include "topology.hpp"
 #include "../../include/mjg.h"
 
@@ -135,6 +136,7 @@ class Batch
         if(const char* a = std::getenv("MJG_AUTOTUNE")) {autotune_ = a[0] != '0';}
         set_lds_limits<float>();
         set_lds_limits<double>();
+        if(transfer_.create(kRepMaxN) != hipSuccess) {throw std::bad_alloc();}
     }
     ~Batch()
     {
@@ -536,16 +538,9 @@ class Batch
     {
         Replica& r = rep(id);
         if(!r.ready) {throw std::logic_error("replica not initialized");}
-        std::vector<double4> h(r.n);
-        double4* src[3] = {r.desc.pos, r.desc.vel, r.desc.force};
+        const double4* src[3] = {r.desc.pos, r.desc.vel, r.desc.force};
         double* dst[3] = {pos, vel, force};
-        for(int k = 0; k < 3; ++k)
-        {
-            if(!dst[k]) {continue;}
-            hip_check(hipMemcpyAsync(h.data(), src[k], r.n * sizeof(double4), hipMemcpyDeviceToHost, stream_), "download");
-            hip_check(hipStreamSynchronize(stream_), "sync");
-            for(size_t i = 0; i < r.n; ++i) {dst[k][3 * i] = h[i].x; dst[k][3 * i + 1] = h[i].y; dst[k][3 * i + 2] = h[i].z;}
-        }
+        hip_check(transfer_.download(src, dst, r.n, stream_), "download");
     }
 
     // forces and per-interaction energies at the current positions (no step)
@@ -1323,6 +1318,7 @@ class Batch
     std::vector<RepState> h_states_;
     std::vector<int> free_slots_;
     std::vector<int> failed_now_;
+    StateTransfer transfer_;
 };
 
 } // mjg

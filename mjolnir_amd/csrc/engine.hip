@@ -44,17 +44,44 @@ void Engine::check(hipError_t e, const char* what)
     }
 }
 
+// Device memory of the engine, freed with it.  Small arrays share chunks: a hipMalloc of its own costs
+// each of an engine's tables about 10 us of set-up.
 template<typename T> T* Engine::dalloc(size_t n)
 {
+    const size_t bytes = (std::max<size_t>(1, n) * sizeof(T) + 255) & ~size_t(255);
+    if(bytes <= chunk_left_)
+    {
+        char* p = chunk_;
+        chunk_ += bytes;
+        chunk_left_ -= bytes;
+        return reinterpret_cast<T*>(p);
+    }
+    const bool share = bytes <= kChunk / 4;
     void* p = nullptr;
-    const size_t bytes = std::max<size_t>(1, n) * sizeof(T);
-    const hipError_t e = hipMalloc(&p, bytes);
+    const hipError_t e = hipMalloc(&p, share ? kChunk : bytes);
     if(e != hipSuccess)
     {
         (void)hipGetLastError();
         throw std::bad_alloc();
     }
     allocations_.push_back(p);
+    if(share)
+    {
+        chunk_ = static_cast<char*>(p) + bytes;
+        chunk_left_ = kChunk - bytes;
+    }
+    return static_cast<T*>(p);
+}
+// pinned host memory that kernels write small results to
+template<typename T> T* Engine::halloc(size_t n)
+{
+    void* p = nullptr;
+    if(hipHostMalloc(&p, n * sizeof(T), hipHostMallocDefault) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        throw std::bad_alloc();
+    }
+    host_allocations_.push_back(p);
     return static_cast<T*>(p);
 }
 template<typename T> void Engine::upload(T* d, const T* h, size_t n)
@@ -101,6 +128,9 @@ Engine::Engine(int precision, int boundary, const double* lower, const double* u
     upload(d_sctl_, &z, 1);
     scratch_n_ = n;
     d_scratch_ = dalloc<double>(n);
+    if(transfer_.create(n) != hipSuccess) {throw std::bad_alloc();}
+    h_energy_ = halloc<double>(kMaxLocalSegs + kMaxGlobals + 2);
+    h_flag_ = reinterpret_cast<int*>(h_energy_ + kMaxLocalSegs + kMaxGlobals + 1);
     // Steps are captured into a hipGraph per segment, except with MJG_NO_GRAPH=1 and under a
     // preloaded profiler library (rocprofv3 preloads librocprofiler-sdk-tool): a kernel-trace run
     // of the graph path once ended in a segmentation fault inside the runtime and the profiler,
@@ -116,6 +146,7 @@ Engine::~Engine()
     if(graph_exec_) {(void)hipGraphExecDestroy(graph_exec_);}
     if(stream_) {(void)hipStreamSynchronize(stream_);}
     for(void* p : allocations_) {(void)hipFree(p);}
+    for(void* p : host_allocations_) {(void)hipHostFree(p);}
     if(stream_) {(void)hipStreamDestroy(stream_);}
 }
 
@@ -145,8 +176,9 @@ void Engine::set_state(const double* mass, const double* pos, const double* vel)
     upload(d_pos_, p.data(), n_);
     upload(d_vel_, v.data(), n_);
     if(d_old_pos_) {upload(d_old_pos_, p.data(), n_);}   // g-BAOAB: the last step end is now
-    std::vector<double4> zf(n_, make_double4(0, 0, 0, 0));
-    upload(d_force_, zf.data(), n_);
+    hipLaunchKernelGGL(k_zero_double4, dim3(blocks_for(n_, 256)), dim3(256), 0, stream_, d_force_, (uint32_t)n_);
+    check(hipGetLastError(), "set_state launch");
+    sync();
     state_set_ = true;
 }
 
@@ -156,32 +188,14 @@ void Engine::set_positions(const double* pos)
 {
     if(!pos) {throw std::invalid_argument("null position pointer");}
     if(!state_set_) {throw std::logic_error("set the state first");}
-    std::vector<double4> p(n_);
-    for(size_t i = 0; i < n_; ++i)
-    {
-        double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
-        if(box_.periodic)
-        {
-            if(x < box_.lower[0]) {x += box_.width[0];} else if(x >= box_.upper[0]) {x -= box_.width[0];}
-            if(y < box_.lower[1]) {y += box_.width[1];} else if(y >= box_.upper[1]) {y -= box_.width[1];}
-            if(z < box_.lower[2]) {z += box_.width[2];} else if(z >= box_.upper[2]) {z -= box_.width[2];}
-        }
-        p[i] = make_double4(x, y, z, 0.0);
-    }
-    upload(d_pos_, p.data(), n_);
+    check(transfer_.upload_positions(pos, d_pos_, n_, box_, stream_), "upload positions");
 }
 
 void Engine::get_state(double* pos, double* vel, double* force)
 {
-    std::vector<double4> h(n_);
-    double4* src[3] = {d_pos_, d_vel_, d_force_};
+    const double4* src[3] = {d_pos_, d_vel_, d_force_};
     double* dst[3] = {pos, vel, force};
-    for(int k = 0; k < 3; ++k)
-    {
-        if(!dst[k]) {continue;}
-        download(h.data(), src[k], n_);
-        for(size_t i = 0; i < n_; ++i) {dst[k][3 * i] = h[i].x; dst[k][3 * i + 1] = h[i].y; dst[k][3 * i + 2] = h[i].z;}
-    }
+    check(transfer_.download(src, dst, n_, stream_), "download");
 }
 
 void Engine::set_attribute(const std::string& key, double value)
@@ -883,7 +897,6 @@ void Engine::initialize()
     d_bak_lctl_ = dalloc<ListCtl>(std::max<size_t>(1, globals_.size()));
     d_abs_margin_ = dalloc<double>(std::max<size_t>(1, globals_.size()));
     d_never_ = dalloc<int>(std::max<size_t>(1, globals_.size()));
-    d_energy_ = dalloc<double>(num_interactions() + 1);
     std::vector<double> absm;
     std::vector<int> never;
     for(auto& g : globals_)
@@ -954,20 +967,20 @@ void Engine::forces(double4* f, bool energy, int only, bool kick, bool advance)
     }
     if(energy)
     {
+        SumSegTable st{};
         for(int l = 0; l < nl; ++l)
         {
             if(only >= 0 && only != l) {continue;}
             const auto& L = locals_[l];
-            hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, stream_, d_te_ + L.term_off, (uint32_t)L.n_terms(),
-                               d_energy_ + l);
+            st.seg[st.n++] = {d_te_ + L.term_off, (uint32_t)L.n_terms(), (uint32_t)l};
         }
         for(size_t gi = 0; gi < globals_.size(); ++gi)
         {
             const int id = nl + (int)gi;
             if(only >= 0 && only != id) {continue;}
-            hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, stream_, globals_[gi].d_epair,
-                               (uint32_t)globals_[gi].part.size(), d_energy_ + id);
+            st.seg[st.n++] = {globals_[gi].d_epair, (uint32_t)globals_[gi].part.size(), (uint32_t)id};
         }
+        if(st.n > 0) {hipLaunchKernelGGL(k_sums, dim3(st.n), dim3(1024), 0, stream_, st, h_energy_);}
     }
     FinishArgs fa{};
     fa.gstart = run_locals ? d_gstart_ : nullptr;
@@ -1082,10 +1095,9 @@ double Engine::calc_force_and_energy()
     if(!initialized_) {throw std::logic_error("not initialized");}
     forces(d_force_, true, -1, false);
     check(hipGetLastError(), "calc_force_and_energy launch");
-    std::vector<double> e(num_interactions());
-    download(e.data(), d_energy_, e.size());
+    sync();
     double tot = 0;
-    for(double x : e) {tot += x;}
+    for(size_t k = 0; k < num_interactions(); ++k) {tot += h_energy_[k];}
     return tot;
 }
 
@@ -1094,10 +1106,9 @@ void Engine::calc_energies(double* per, double* total)
     if(!initialized_) {throw std::logic_error("not initialized");}
     forces(d_force_tmp_, true, -1, false);
     check(hipGetLastError(), "calc_energies launch");
-    std::vector<double> e(num_interactions());
-    download(e.data(), d_energy_, e.size());
+    sync();
     double tot = 0;
-    for(size_t k = 0; k < e.size(); ++k) {if(per) {per[k] = e[k];} tot += e[k];}
+    for(size_t k = 0; k < num_interactions(); ++k) {if(per) {per[k] = h_energy_[k];} tot += h_energy_[k];}
     if(total) {*total = tot;}
 }
 
@@ -1107,27 +1118,21 @@ void Engine::calc_force_of(int id, double* out)
     if(id < 0 || (size_t)id >= num_interactions()) {throw std::out_of_range("interaction id out of range");}
     forces(d_force_tmp_, false, id, false);
     check(hipGetLastError(), "calc_force_of launch");
-    std::vector<double4> h(n_);
-    download(h.data(), d_force_tmp_, n_);
-    for(size_t i = 0; i < n_; ++i) {out[3 * i] = h[i].x; out[3 * i + 1] = h[i].y; out[3 * i + 2] = h[i].z;}
+    const double4* src[3] = {d_force_tmp_, nullptr, nullptr};
+    double* dst[3] = {out, nullptr, nullptr};
+    check(transfer_.download(src, dst, n_, stream_), "download");
 }
 
 void Engine::reduce_margin(double dmargin)
 {
     if(!initialized_) {throw std::logic_error("not initialized");}
     if(globals_.empty()) {return;}
-    std::vector<ListCtl> ctl(globals_.size());
-    download(ctl.data(), d_lctl_, globals_.size());
-    bool any = false;
-    for(size_t g = 0; g < globals_.size(); ++g)
-    {
-        if(globals_[g].partition == MJG_PART_NAIVE) {continue;}
-        ctl[g].margin -= dmargin;
-        any = any || ctl[g].margin < 0;
-    }
-    upload(d_lctl_, ctl.data(), globals_.size());
+    hipLaunchKernelGGL(k_reduce_margin, dim3(1), dim3(64), 0, stream_, d_lctl_, d_never_, (uint32_t)globals_.size(),
+                       dmargin, h_flag_);
+    check(hipGetLastError(), "reduce_margin launch");
+    sync();
     // a rebuild resets the margin of every list (rebuilding a list early is always valid)
-    if(any) {build_lists_now(true);}
+    if(*h_flag_) {build_lists_now(true);}
 }
 
 size_t Engine::neighbor_pairs(int id, uint32_t* pairs, size_t cap)
@@ -1614,10 +1619,11 @@ double Engine::kinetic_energy()
 {
     hipLaunchKernelGGL(k_kinetic, dim3(blocks_for(n_, 256)), dim3(256), 0, stream_, (uint32_t)n_, d_vel_, d_mass_,
                        d_scratch_);
-    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, stream_, d_scratch_, (uint32_t)n_, d_energy_ + num_interactions());
+    double* out = h_energy_ + kMaxLocalSegs + kMaxGlobals;
+    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, stream_, d_scratch_, (uint32_t)n_, out);
     check(hipGetLastError(), "kinetic launch");
-    double ke = 0;
-    download(&ke, d_energy_ + num_interactions(), 1);
+    sync();
+    const double ke = *out;
     return ke;
 }
 

@@ -6,9 +6,11 @@
 #include "force_kernels.hpp"
 #include "integrate_kernels.hpp"
 #include "constraint_kernels.hpp"
+#include "host_io.hpp"
 #include "nlist_kernels.hpp"
 #include "tile_kernels.hpp"
 
+#include <algorithm>
 #include <map>
 #include <stdexcept>
 #include <string>
@@ -156,6 +158,7 @@ class Engine
     void sync();
     void check(hipError_t e, const char* what);
     template<typename T> T* dalloc(size_t n);
+    template<typename T> T* halloc(size_t n);
     template<typename T> void upload(T* d, const T* h, size_t n);
     template<typename T> void download(T* h, const T* d, size_t n);
 
@@ -163,7 +166,13 @@ class Engine
     size_t n_;
     Box box_{};
     hipStream_t stream_ = nullptr;
-    std::vector<void*> allocations_;
+    StateTransfer transfer_;
+    double* h_energy_ = nullptr;   // pinned: per interaction, then the kinetic energy
+    int* h_flag_ = nullptr;        // pinned: a kernel's decision for the host
+    std::vector<void*> allocations_, host_allocations_;
+    static constexpr size_t kChunk = size_t(1) << 18;   // shared chunk of small device arrays
+    char* chunk_ = nullptr;                              // its unused rest
+    size_t chunk_left_ = 0;
 
     std::vector<double> mass_;
     bool has_T_ = false, has_I_ = false, initialized_ = false, integ_ready_ = false, state_set_ = false;
@@ -218,7 +227,6 @@ class Engine
     ListCtl* d_bak_lctl_ = nullptr;
     double* d_abs_margin_ = nullptr;
     int* d_never_ = nullptr;
-    double* d_energy_ = nullptr;    // per interaction + total
     double* d_scratch_ = nullptr;   // N doubles
     size_t scratch_n_ = 0;
 

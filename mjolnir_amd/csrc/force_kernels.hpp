@@ -711,14 +711,34 @@ __global__ void k_zero_double4(double4* __restrict__ p, uint32_t n)
 
 // Deterministic sum of n doubles (one block of 1024 threads): thread k adds elements
 // k, k+1024, ... in order, then a fixed-shape tree.
-__global__ void __launch_bounds__(1024)
-k_sum(const double* __restrict__ in, uint32_t n, double* __restrict__ out)
+__device__ __forceinline__ void sum_to(const double* __restrict__ in, uint32_t n, double* __restrict__ out)
 {
     __shared__ double lds[16];
     double s = 0.0;
     for(uint32_t k = threadIdx.x; k < n; k += blockDim.x) {s += in[k];}
     s = block_sum(s, lds);
     if(threadIdx.x == 0) {*out = s;}
+}
+__global__ void __launch_bounds__(1024)
+k_sum(const double* __restrict__ in, uint32_t n, double* __restrict__ out) {sum_to(in, n, out);}
+
+// The energies of every interaction in one launch, a block each (one launch a sum before).
+struct SumSeg
+{
+    const double* in;
+    uint32_t n;
+    uint32_t id;       // out[id] takes the sum
+};
+struct SumSegTable
+{
+    SumSeg seg[kMaxLocalSegs + kMaxPairSegs];
+    int n;
+};
+__global__ void __launch_bounds__(1024)
+k_sums(SumSegTable t, double* __restrict__ out)
+{
+    const SumSeg& s = t.seg[blockIdx.x];
+    sum_to(s.in, s.n, out + s.id);
 }
 
 } // mjg

@@ -55,6 +55,24 @@ struct ListCtl
     double margin;                 // current_margin of the partition
 };
 
+// ForceField::reduce_margin (ForceField.hpp:75-92) called from the host: every list's margin less
+// dmargin; *spent (pinned host memory) tells whether one ran out.  One thread per interaction of a
+// single wave.
+__global__ void __launch_bounds__(64)
+k_reduce_margin(ListCtl* __restrict__ ctl, const int* __restrict__ never, uint32_t n, double dmargin,
+                int* __restrict__ spent)
+{
+    bool out = false;
+    if(threadIdx.x < n && !never[threadIdx.x])
+    {
+        const double m = ctl[threadIdx.x].margin - dmargin;
+        ctl[threadIdx.x].margin = m;
+        out = m < 0;
+    }
+    const bool any = __any(out);
+    if(threadIdx.x == 0) {*spent = any ? 1 : 0;}
+}
+
 __global__ void k_bbox(const double4* __restrict__ pos, const uint32_t* __restrict__ part, uint32_t np,
                        ListCtl* __restrict__ ctl)
 {
