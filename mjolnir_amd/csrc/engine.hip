@@ -129,8 +129,12 @@ Engine::Engine(int precision, int boundary, const double* lower, const double* u
     scratch_n_ = n;
     d_scratch_ = dalloc<double>(n);
     if(transfer_.create(n) != hipSuccess) {throw std::bad_alloc();}
-    h_energy_ = halloc<double>(kMaxLocalSegs + kMaxGlobals + 2);
+    // pinned results: energies, flag, step control, list control
+    static_assert(sizeof(StepCtl) % 8 == 0 && sizeof(ListCtl) % 8 == 0, "pinned results are laid out in words");
+    h_energy_ = halloc<double>(kMaxLocalSegs + kMaxGlobals + 2 + (sizeof(StepCtl) + kMaxGlobals * sizeof(ListCtl)) / 8);
     h_flag_ = reinterpret_cast<int*>(h_energy_ + kMaxLocalSegs + kMaxGlobals + 1);
+    h_sctl_ = reinterpret_cast<StepCtl*>(h_energy_ + kMaxLocalSegs + kMaxGlobals + 2);
+    h_lctl_ = reinterpret_cast<ListCtl*>(h_sctl_ + 1);
     // Steps are captured into a hipGraph per segment, except with MJG_NO_GRAPH=1 and under a
     // preloaded profiler library (rocprofv3 preloads librocprofiler-sdk-tool): a kernel-trace run
     // of the graph path once ended in a segmentation fault inside the runtime and the profiler,
@@ -474,6 +478,9 @@ static uint32_t tile_min_np()
     return kTileMinNp;
 }
 
+// Largest interaction whose list k_forces keeps by brute force (np^2 / 2 distance tests a rebuild).
+constexpr size_t kSelfMaxPart = 4096;
+
 // lanes per participant: about six partners per lane, a power of two in [1, 64]
 static uint32_t lanes_for(uint32_t maxcount)
 {
@@ -620,7 +627,6 @@ void Engine::setup_global(GlobalIA& g)
         }
     }
     g.d_nn = dalloc<uint32_t>(np);
-    g.d_order = dalloc<uint32_t>(np);
     g.d_spart = dalloc<uint32_t>(np);
     if(g.partition == MJG_PART_CELLLIST) {g.d_spos = dalloc<double4>(np);}
     g.d_epair = dalloc<double>(np);
@@ -652,7 +658,6 @@ ListSeg Engine::list_seg(GlobalIA& g, size_t gi)
     s.nl = g.d_nl;
     s.nl16 = g.tiled ? g.d_nl16 : nullptr;
     s.nn = g.d_nn;
-    s.order = g.d_order;
     s.spart = g.d_spart;
     s.spos = g.d_spos;
     s.ctl = d_lctl_ + gi;
@@ -695,8 +700,7 @@ PairSegTable Engine::pair_table(int only)
         s.np = (uint32_t)g.part.size();
         s.block_begin = block;
         s.cap = g.cap;
-        s.part = g.d_part;
-        s.order = g.d_order;
+        s.spart = g.d_spart;
         s.nl = g.d_nl;
         s.nn = g.d_nn;
         s.ppar = g.d_ppar;
@@ -711,7 +715,7 @@ PairSegTable Engine::pair_table(int only)
 // Launch the skin check and the rebuild pipeline of every global interaction; the kernels
 // check ListCtl::rebuild themselves, so a captured step always launches the same sequence.
 // force != 0 rebuilds every list now (initialize, explicit reduce_margin, capacity growth).
-void Engine::launch_rebuilds(int force)
+void Engine::launch_rebuilds(int force, uint32_t k)
 {
     PrepSegTable small{}, large{};
     std::vector<int> large_ids;
@@ -737,11 +741,11 @@ void Engine::launch_rebuilds(int force)
     }
     if(small.n > 0)
     {
-        hipLaunchKernelGGL(k_prep_small, dim3(small.n), dim3(1024), 0, stream_, d_pos_, small, d_sctl_, force);
+        hipLaunchKernelGGL(k_prep_small, dim3(small.n), dim3(1024), 0, stream_, d_pos_, small, d_sctl_, k, force);
     }
     if(large.n > 0)
     {
-        hipLaunchKernelGGL(k_margin_large, dim3(1), dim3(64), 0, stream_, large, d_sctl_, force);
+        hipLaunchKernelGGL(k_margin_large, dim3(1), dim3(64), 0, stream_, large, d_sctl_, k, force);
         for(int gi : large_ids)
         {
             GlobalIA& g = globals_[gi];
@@ -824,7 +828,7 @@ void Engine::build_lists_now(bool)
     download(ctl.data(), d_lctl_, globals_.size());
     for(auto& c : ctl) {c.rebuild = 0;}
     upload(d_lctl_, ctl.data(), globals_.size());
-    grow_tiles();
+    grow_tiles(ctl);
 }
 
 void Engine::initialize()
@@ -845,7 +849,7 @@ void Engine::initialize()
                               (int)((size_t)kTileMaxCap * kBuildBytesPerParticle)), "tile attribute");
     write_topology();
 
-    // local tables: one segment per interaction, body slots in interaction/term/body order
+    // local tables: one segment per interaction
     std::vector<uint32_t> lidx;
     std::vector<double> lpar;
     std::vector<std::vector<uint32_t>> per_particle(n_);
@@ -878,19 +882,21 @@ void Engine::initialize()
     n_terms_ = term;
     if(!locals_.empty())
     {
-        std::vector<uint32_t> gstart(n_ + 1), gslot;
+        // a particle's slots lie one after the other; tdst is the slot of each term's body
+        std::vector<uint32_t> gstart(n_ + 1), tdst(n_slots_);
+        uint32_t at = 0;
         for(size_t i = 0; i < n_; ++i)
         {
-            gstart[i] = (uint32_t)gslot.size();
-            gslot.insert(gslot.end(), per_particle[i].begin(), per_particle[i].end());
+            gstart[i] = at;
+            for(uint32_t body : per_particle[i]) {tdst[body] = at++;}
         }
-        gstart[n_] = (uint32_t)gslot.size();
+        gstart[n_] = at;
         d_lidx_ = dalloc<uint32_t>(lidx.size()); upload(d_lidx_, lidx.data(), lidx.size());
         d_lpar_ = dalloc<double>(lpar.size()); upload(d_lpar_, lpar.data(), lpar.size());
         d_tf_ = dalloc<double>(3 * (size_t)n_slots_);
         d_te_ = dalloc<double>(n_terms_);
         d_gstart_ = dalloc<uint32_t>(n_ + 1); upload(d_gstart_, gstart.data(), n_ + 1);
-        d_gslot_ = dalloc<uint32_t>(gslot.size()); upload(d_gslot_, gslot.data(), gslot.size());
+        d_tdst_ = dalloc<uint32_t>(tdst.size()); upload(d_tdst_, tdst.data(), tdst.size());
     }
 
     d_lctl_ = dalloc<ListCtl>(std::max<size_t>(1, globals_.size()));
@@ -913,14 +919,24 @@ void Engine::initialize()
         upload(d_lctl_, ctl.data(), ctl.size());
         build_lists_now(true);
     }
+    for(const auto& L : locals_)
+    {
+        tsp_ = tsp_ || L.kind == kBond3SPN2 || L.kind == kDihedralPGauss || L.kind == kBaseStacking;
+    }
+    small_ = !globals_.empty() && globals_.size() <= (size_t)kMaxSelfLists && locals_.size() <= (size_t)kMaxSmallLocals &&
+             n_ <= 4 * (size_t)kSelfMaxPart;
+    for(const auto& g : globals_)
+    {
+        tsp_ = tsp_ || g.multibody() || g.pot == kPair3SPN2EV;
+        small_ = small_ && !g.tiled && g.part.size() <= kSelfMaxPart;
+    }
+    if(small_) {d_noise_ = dalloc<double4>(n_);}
     initialized_ = true;
 }
 
-// ForceField::calc_force into f: locals (term kernel), every pair interaction (fused kernel),
-// then k_finish sums them per particle (and with `kick` applies the closing half-kick of the
-// integrator step).  With `energy`, per-interaction energies land in d_energy_.  only >= 0
-// restricts the call to one interaction id.
-void Engine::forces(double4* f, bool energy, int only, bool kick, bool advance)
+// Every interaction's forces (local terms into their slots, pair interactions into their arrays), and
+// with `energy` the energies into h_energy_.  only >= 0 restricts the call to one interaction id.
+void Engine::interaction_forces(bool energy, int only)
 {
     const int nl = (int)locals_.size();
     const bool run_locals = local_blocks_ > 0 && (only < 0 || only < nl);
@@ -935,12 +951,12 @@ void Engine::forces(double4* f, bool energy, int only, bool kick, bool advance)
         if(energy)
         {
             hipLaunchKernelGGL(k_local_terms<true>, dim3(local_blocks_), dim3(256), 0, stream_, d_pos_, box_, segtab_,
-                               d_lidx_, d_lpar_, d_tf_, d_te_, only);
+                               d_lidx_, d_lpar_, d_tdst_, d_tf_, d_te_, only);
         }
         else
         {
             hipLaunchKernelGGL(k_local_terms<false>, dim3(local_blocks_), dim3(256), 0, stream_, d_pos_, box_, segtab_,
-                               d_lidx_, d_lpar_, d_tf_, d_te_, only);
+                               d_lidx_, d_lpar_, d_tdst_, d_tf_, d_te_, only);
         }
     }
     const PairSegTable pt = pair_table(only);
@@ -982,16 +998,31 @@ void Engine::forces(double4* f, bool energy, int only, bool kick, bool advance)
         }
         if(st.n > 0) {hipLaunchKernelGGL(k_sums, dim3(st.n), dim3(1024), 0, stream_, st, h_energy_);}
     }
-    FinishArgs fa{};
-    fa.gstart = run_locals ? d_gstart_ : nullptr;
-    fa.gslot = d_gslot_;
-    fa.tf = d_tf_;
-    fa.ng = 0;
+}
+
+GatherArgs Engine::gather_args(bool locals, int only, bool sums)
+{
+    GatherArgs a{};
+    a.gstart = locals ? d_gstart_ : nullptr;
+    a.tf = d_tf_;
     for(size_t gi = 0; gi < globals_.size(); ++gi)
     {
-        if(only >= 0 && only != nl + (int)gi) {continue;}
-        fa.fg[fa.ng++] = globals_[gi].d_fg;
+        if(only >= 0 && only != (int)(locals_.size() + gi)) {continue;}
+        const bool acc = sums && globals_[gi].multibody();
+        a.fg[a.ng] = acc ? nullptr : globals_[gi].d_fg;
+        a.acc[a.ng] = acc ? globals_[gi].d_acc : nullptr;
+        ++a.ng;
     }
+    return a;
+}
+
+// ForceField::calc_force into f: the interactions' forces, then k_finish sums them per particle
+// (and with `kick` applies the closing half-kick of the integrator step).
+void Engine::forces(double4* f, bool energy, int only, bool kick, bool advance)
+{
+    interaction_forces(energy, only);
+    FinishArgs fa{};
+    fa.g = gather_args(local_blocks_ > 0 && (only < 0 || only < (int)locals_.size()), only, false);
     fa.halfdt = dt_ / 2;
     fa.kick = kick ? 1 : 0;
     fa.advance = (kick || advance) ? 1 : 0;
@@ -1008,7 +1039,7 @@ void Engine::launch_multibody(const GlobalIA& g, bool energy)
                        (uint32_t)(3 * n_ + 1));
     TspSeg s{};
     s.kind = g.pot; s.np = np; s.cap = g.cap; s.tpp = g.mb_tpp;
-    s.part = g.d_part; s.order = g.d_order; s.nl = g.d_nl; s.nn = g.d_nn;
+    s.spart = g.d_spart; s.nl = g.d_nl; s.nn = g.d_nn;
     s.ppar = g.d_ppar; s.acc = g.d_acc; s.n = (uint32_t)n_; s.eout = g.d_epair;
     const uint32_t blocks = blocks_for((size_t)np * s.tpp, 256);
     if(energy) {hipLaunchKernelGGL(k_tsp_pairs<true>, dim3(blocks), dim3(256), 0, stream_, d_pos_, box_, s);}
@@ -1023,7 +1054,7 @@ void Engine::launch_tiled(GlobalIA& g, int gi, bool energy)
     TileSeg s{};
     PairSeg& ps = s.ps;
     ps.kind = g.pot; ps.tpp = g.tpp; ps.np = (uint32_t)g.part.size(); ps.block_begin = 0; ps.cap = g.cap;
-    ps.part = g.d_part; ps.order = g.d_order; ps.nl = g.d_nl; ps.nn = g.d_nn; ps.ppar = g.d_ppar;
+    ps.spart = g.d_spart; ps.nl = g.d_nl; ps.nn = g.d_nn; ps.ppar = g.d_ppar;
     ps.fout = g.d_fg; ps.eout = g.d_epair; ps.pp = g.pp;
     s.nl16 = g.d_nl16; s.spart = g.d_spart; s.cell_start = g.d_cell_start; s.cell_end = g.d_cell_end;
     s.grid = g.d_grid; s.ctl = d_lctl_ + gi; s.cap_nbr = g.tile_cap;
@@ -1061,16 +1092,13 @@ uint32_t Engine::tile_lanes(const GlobalIA& g) const
 // After lists were built: a tiled interaction whose largest neighbourhood outgrew its staging
 // capacity gets a larger one (its launches served that build from global memory meanwhile).
 // True if a capacity changed, which invalidates a captured step graph.
-bool Engine::grow_tiles()
+bool Engine::grow_tiles(const std::vector<ListCtl>& ctl)
 {
     bool any = false;
-    std::vector<ListCtl> ctl(globals_.size());
-    bool have = false;
     for(size_t gi = 0; gi < globals_.size(); ++gi)
     {
         GlobalIA& g = globals_[gi];
         if(!g.tiled) {continue;}
-        if(!have) {download(ctl.data(), d_lctl_, globals_.size()); have = true;}
         const uint32_t need = ctl[gi].maxnbr;
         if(need > g.tile_cap && g.tile_cap < kTileMaxCap && !g.tile_fixed)
         {
@@ -1142,14 +1170,14 @@ size_t Engine::neighbor_pairs(int id, uint32_t* pairs, size_t cap)
     if(gi < 0 || (size_t)gi >= globals_.size()) {throw std::out_of_range("not a global interaction id");}
     GlobalIA& g = globals_[gi];
     const uint32_t np = (uint32_t)g.part.size();
-    std::vector<uint32_t> nn(np), order(np), nl((size_t)np * g.cap);
+    std::vector<uint32_t> nn(np), spart(np), nl((size_t)np * g.cap);
     download(nn.data(), g.d_nn, np);
-    download(order.data(), g.d_order, np);
+    download(spart.data(), g.d_spart, np);
     download(nl.data(), g.d_nl, nl.size());
     std::vector<std::pair<uint32_t, uint32_t>> out;
     for(uint32_t t = 0; t < np; ++t)
     {
-        const uint32_t i = g.part[order[t]];
+        const uint32_t i = spart[t];
         for(uint32_t k = 0; k < nn[t]; ++k)
         {
             const uint32_t j = nl[(size_t)t * g.cap + k];
@@ -1374,31 +1402,167 @@ void Engine::launch_step()
     }
     if(!globals_.empty()) {launch_rebuilds(0);}
     forces(d_force_, false, -1, true);
-    if(rm_translation_ || rm_rotation_)
+    hipLaunchKernelGGL(k_remove_motion, dim3(1), dim3(kRemoverThreads), 0, stream_, (uint32_t)n_, d_pos_, d_vel_,
+                       d_mass_, rm_translation_, rm_rotation_, rm_rescale_);
+}
+
+// Whether consecutive steps are joined by k_advance: BAOAB and G-JF without a motion remover, which
+// would have to run between the closing kick and the next step.
+bool Engine::advances() const
+{
+    return (integ_ == MJG_INTEG_BAOAB || integ_ == MJG_INTEG_GJF) && !rm_translation_ && !rm_rotation_;
+}
+
+// k_advance in front of step k of the segment (k = 0: its start), or closing it after k steps.
+void Engine::launch_advance(uint32_t k, bool last)
+{
+    AdvanceArgs a{};
+    a.g = gather_args(local_blocks_ > 0, -1, small_);
+    if(small_)
     {
-        hipLaunchKernelGGL(k_remove_motion, dim3(1), dim3(kRemoverThreads), 0, stream_, (uint32_t)n_, d_pos_, d_vel_,
-                           d_mass_, rm_translation_, rm_rotation_, rm_rescale_);
+        for(size_t gi = 0; gi < globals_.size(); ++gi)
+        {
+            a.lists.ctl[gi] = d_lctl_ + gi;
+            a.lists.abs_margin[gi] = globals_[gi].max_cutoff * globals_[gi].margin;
+            a.lists.never[gi] = (globals_[gi].partition == MJG_PART_NAIVE);
+        }
+        a.lists.n = (int)globals_.size();
+        a.noise = d_noise_;
     }
+    a.pos = d_pos_; a.vel = d_vel_; a.force = d_force_;
+    a.rmass = d_rmass_; a.c1 = d_c1_; a.c2 = d_c2_; a.c3 = d_c3_;
+    a.ctl = d_sctl_;
+    a.lctl = d_lctl_; a.h_lctl = h_lctl_; a.h_ctl = h_sctl_;
+    a.nlists = (int)globals_.size();
+    a.dt = dt_; a.halfdt = dt_ / 2;
+    a.seed = seed_;
+    a.box = box_;
+    a.n = (uint32_t)n_;
+    a.k = k;
+    const dim3 grid(blocks_for(n_, 256)), block(256);
+    const bool gjf = (integ_ == MJG_INTEG_GJF);
+    if(k == 0)
+    {
+        if(gjf) {hipLaunchKernelGGL((k_advance<true, true, false>), grid, block, 0, stream_, a);}
+        else {hipLaunchKernelGGL((k_advance<false, true, false>), grid, block, 0, stream_, a);}
+    }
+    else if(last)
+    {
+        if(gjf) {hipLaunchKernelGGL((k_advance<true, false, true>), grid, block, 0, stream_, a);}
+        else {hipLaunchKernelGGL((k_advance<false, false, true>), grid, block, 0, stream_, a);}
+    }
+    else
+    {
+        if(gjf) {hipLaunchKernelGGL((k_advance<true, false, false>), grid, block, 0, stream_, a);}
+        else {hipLaunchKernelGGL((k_advance<false, false, false>), grid, block, 0, stream_, a);}
+    }
+}
+
+// The forces of step k: one launch for a small system, else the rebuild pipeline and the
+// interactions' own kernels.
+void Engine::launch_step_forces(uint32_t k)
+{
+    if(!small_)
+    {
+        if(!globals_.empty()) {launch_rebuilds(0, k);}
+        interaction_forces(false, -1);
+        return;
+    }
+    SmallForces a{};
+    uint32_t block = 0;
+    // 3SPN2 rows first: theirs are the longest chains of arithmetic
+    for(int pass = 0; pass < 2; ++pass)
+    {
+        for(size_t gi = 0; gi < globals_.size(); ++gi)
+        {
+            GlobalIA& g = globals_[gi];
+            if(g.multibody() != (pass == 0)) {continue;}
+            RowSeg& r = a.row[a.nrow++];
+            r.block_begin = block;
+            r.never = (g.partition == MJG_PART_NAIVE);
+            r.p.kind = g.pot; r.p.tpp = g.multibody() ? g.mb_tpp : g.tpp; r.p.np = (uint32_t)g.part.size(); r.p.cap = g.cap;
+            r.p.spart = g.d_spart; r.p.nl = g.d_nl; r.p.nn = g.d_nn; r.p.ppar = g.d_ppar; r.p.fout = g.d_fg;
+            r.p.pp = g.pp;
+            r.acc = g.d_acc;
+            r.ctl = d_lctl_ + gi;
+            r.nl = g.d_nl; r.nn = g.d_nn;
+            r.part = g.d_part; r.pslot = g.d_pslot; r.mol = g.d_mol; r.ex_start = g.d_ex_start; r.ex = g.d_ex;
+            r.rule = g.rule;
+            block += blocks_for((size_t)r.p.np * r.p.tpp, 256);
+        }
+    }
+    a.local_begin = block;
+    a.nlocal = segtab_.n;
+    for(int l = 0; l < segtab_.n; ++l) {a.local[l] = segtab_.seg[l];}
+    block += local_blocks_;
+    a.noise_begin = block;
+    block += blocks_for(n_, 256);
+    a.lidx = d_lidx_; a.lpar = d_lpar_; a.ldst = d_tdst_; a.tf = d_tf_;
+    a.noise = d_noise_; a.seed = seed_; a.sctl = d_sctl_; a.n = (uint32_t)n_; a.k = k;
+    const bool mixed = (precision_ == MJG_FP32_FIXED);
+    const dim3 grid(block), threads(256);
+    if(mixed && tsp_) {hipLaunchKernelGGL((k_forces<true, true>), grid, threads, 0, stream_, d_pos_, box_, a);}
+    else if(mixed) {hipLaunchKernelGGL((k_forces<true, false>), grid, threads, 0, stream_, d_pos_, box_, a);}
+    else if(tsp_) {hipLaunchKernelGGL((k_forces<false, true>), grid, threads, 0, stream_, d_pos_, box_, a);}
+    else {hipLaunchKernelGGL((k_forces<false, false>), grid, threads, 0, stream_, d_pos_, box_, a);}
+}
+
+// A segment of n joined steps: its start saved, n steps, and the control words sent to the host.
+void Engine::launch_segment(size_t n)
+{
+    BackupArgs b{};
+    b.src[0] = d_pos_; b.src[1] = d_vel_; b.src[2] = d_force_;
+    b.dst[0] = d_bak_pos_; b.dst[1] = d_bak_vel_; b.dst[2] = d_bak_force_;
+    b.ctl = d_sctl_; b.bak_ctl = d_bak_sctl_;
+    b.lctl = d_lctl_; b.bak_lctl = d_bak_lctl_;
+    b.n = (uint32_t)n_;
+    b.nlists = (int)globals_.size();
+    hipLaunchKernelGGL(k_backup, dim3(std::min<uint32_t>(blocks_for(n_, 256), 2048)), dim3(256), 0, stream_, b);
+    if(small_)
+    {
+        // the multibody sums start at zero; k_advance clears what it has read
+        for(const auto& g : globals_)
+        {
+            if(!g.multibody()) {continue;}
+            hipLaunchKernelGGL(k_zero_u64, dim3(blocks_for(3 * n_ + 1, 256)), dim3(256), 0, stream_, g.d_acc,
+                               (uint32_t)(3 * n_ + 1));
+        }
+    }
+    for(size_t k = 0; k < n; ++k)
+    {
+        launch_advance((uint32_t)k, false);
+        launch_step_forces((uint32_t)k);
+    }
+    launch_advance((uint32_t)n, true);
 }
 
 void Engine::run_segment(size_t n)
 {
     const size_t ng = std::max<size_t>(1, globals_.size());
+    const bool joined = advances();
     for(int attempt = 0; attempt < 6; ++attempt)
     {
-        check(hipMemcpyAsync(d_bak_pos_, d_pos_, n_ * sizeof(double4), hipMemcpyDeviceToDevice, stream_), "backup");
-        check(hipMemcpyAsync(d_bak_vel_, d_vel_, n_ * sizeof(double4), hipMemcpyDeviceToDevice, stream_), "backup");
-        check(hipMemcpyAsync(d_bak_force_, d_force_, n_ * sizeof(double4), hipMemcpyDeviceToDevice, stream_), "backup");
-        check(hipMemcpyAsync(d_bak_sctl_, d_sctl_, sizeof(StepCtl), hipMemcpyDeviceToDevice, stream_), "backup");
-        if(integ_ == MJG_INTEG_UNDERDAMPED)
+        if(!joined)
         {
-            check(hipMemcpyAsync(d_bak_accel_, d_accel_, n_ * sizeof(double4), hipMemcpyDeviceToDevice, stream_),
-                  "backup");
+            check(hipMemcpyAsync(d_bak_pos_, d_pos_, n_ * sizeof(double4), hipMemcpyDeviceToDevice, stream_), "backup");
+            check(hipMemcpyAsync(d_bak_vel_, d_vel_, n_ * sizeof(double4), hipMemcpyDeviceToDevice, stream_), "backup");
+            check(hipMemcpyAsync(d_bak_force_, d_force_, n_ * sizeof(double4), hipMemcpyDeviceToDevice, stream_), "backup");
+            check(hipMemcpyAsync(d_bak_sctl_, d_sctl_, sizeof(StepCtl), hipMemcpyDeviceToDevice, stream_), "backup");
+            if(integ_ == MJG_INTEG_UNDERDAMPED)
+            {
+                check(hipMemcpyAsync(d_bak_accel_, d_accel_, n_ * sizeof(double4), hipMemcpyDeviceToDevice, stream_),
+                      "backup");
+            }
+            if(!globals_.empty())
+            {
+                check(hipMemcpyAsync(d_bak_lctl_, d_lctl_, ng * sizeof(ListCtl), hipMemcpyDeviceToDevice, stream_),
+                      "backup");
+            }
         }
-        if(!globals_.empty())
-        {
-            check(hipMemcpyAsync(d_bak_lctl_, d_lctl_, ng * sizeof(ListCtl), hipMemcpyDeviceToDevice, stream_), "backup");
-        }
+        auto launch = [&]() {
+            if(joined) {launch_segment(n);}
+            else {for(size_t s = 0; s < n; ++s) {launch_step();}}
+        };
         if(use_graph_)
         {
             if(graph_exec_ == nullptr || graph_steps_ != n)
@@ -1406,7 +1570,7 @@ void Engine::run_segment(size_t n)
                 if(graph_exec_) {(void)hipGraphExecDestroy(graph_exec_); graph_exec_ = nullptr;}
                 hipGraph_t graph = nullptr;
                 check(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "begin capture");
-                for(size_t s = 0; s < n; ++s) {launch_step();}
+                launch();
                 check(hipStreamEndCapture(stream_, &graph), "end capture");
                 check(hipGraphInstantiate(&graph_exec_, graph, nullptr, nullptr, 0), "graph instantiate");
                 (void)hipGraphDestroy(graph);
@@ -1416,29 +1580,35 @@ void Engine::run_segment(size_t n)
         }
         else
         {
-            for(size_t s = 0; s < n; ++s) {launch_step();}
+            launch();
             check(hipGetLastError(), "step launch");
         }
         StepCtl sc{};
-        download(&sc, d_sctl_, 1);
-        bool overflow = false;
-        if(!globals_.empty())
+        std::vector<ListCtl> ctl(globals_.size());
+        if(joined)
         {
-            std::vector<ListCtl> ctl(globals_.size());
-            download(ctl.data(), d_lctl_, globals_.size());
-            for(size_t g = 0; g < globals_.size(); ++g)
+            sync();
+            sc = *h_sctl_;
+            std::copy(h_lctl_, h_lctl_ + globals_.size(), ctl.begin());
+        }
+        else
+        {
+            download(&sc, d_sctl_, 1);
+            if(!globals_.empty()) {download(ctl.data(), d_lctl_, globals_.size());}
+        }
+        bool overflow = false;
+        for(size_t g = 0; g < globals_.size(); ++g)
+        {
+            if(ctl[g].maxcount > globals_[g].cap)
             {
-                if(ctl[g].maxcount > globals_[g].cap)
-                {
-                    alloc_list(globals_[g], (uint32_t)(ctl[g].maxcount + ctl[g].maxcount / 4 + 16));
-                    overflow = true;
-                }
+                alloc_list(globals_[g], (uint32_t)(ctl[g].maxcount + ctl[g].maxcount / 4 + 16));
+                overflow = true;
             }
         }
         if(!overflow)
         {
             if(sc.nonfinite) {throw NonFinite("non-finite particle position");}
-            grow_tiles();
+            grow_tiles(ctl);
             return;
         }
         // a partner list did not fit: restore the segment's start, force a rebuild with the
@@ -1700,7 +1870,7 @@ double Engine::profile_interaction(int id, int reps, uint64_t* half_pairs)
         if(id < nl)
         {
             hipLaunchKernelGGL(k_local_terms<false>, dim3(local_blocks_), dim3(256), 0, stream_, d_pos_, box_, segtab_,
-                               d_lidx_, d_lpar_, d_tf_, d_te_, id);
+                               d_lidx_, d_lpar_, d_tdst_, d_tf_, d_te_, id);
         }
         else if(globals_[id - nl].multibody()) {launch_multibody(globals_[id - nl], false);}
         else if(globals_[id - nl].tiled) {launch_tiled(globals_[id - nl], id - nl, false);}

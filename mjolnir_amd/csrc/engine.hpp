@@ -8,6 +8,7 @@
 #include "constraint_kernels.hpp"
 #include "host_io.hpp"
 #include "nlist_kernels.hpp"
+#include "step_kernels.hpp"
 #include "tile_kernels.hpp"
 
 #include <algorithm>
@@ -60,7 +61,7 @@ struct GlobalIA
     Grid* d_grid = nullptr;
     CellSort sb;
     uint32_t *d_cell_start = nullptr, *d_cell_end = nullptr;
-    uint32_t *d_nl = nullptr, *d_nn = nullptr, *d_order = nullptr, *d_spart = nullptr;
+    uint32_t *d_nl = nullptr, *d_nn = nullptr, *d_spart = nullptr;
     double4* d_spos = nullptr;    // position of each sorted slot at the last cell-list build
     uint32_t cap = 0;             // row length of the list: nl[t * cap + k]
     uint32_t tpp = 8;             // lanes per participant in k_verlet / k_pairs
@@ -141,14 +142,20 @@ class Engine
     void make_exclusions(GlobalIA& g);
     void setup_global(GlobalIA& g);
     void alloc_list(GlobalIA& g, uint32_t cap);
-    void launch_rebuilds(int force);
+    void launch_rebuilds(int force, uint32_t k = 0);
+    GatherArgs gather_args(bool locals, int only, bool sums);
+    bool advances() const;
+    void launch_advance(uint32_t k, bool last);
+    void launch_step_forces(uint32_t k);
+    void launch_segment(size_t n);
+    void interaction_forces(bool energy, int only);
     void build_lists_now(bool all);
     ListSeg list_seg(GlobalIA& g, size_t gi);
     ListSegTable list_table();
     PairSegTable pair_table(int only);
     void launch_multibody(const GlobalIA& g, bool energy);
     void launch_tiled(GlobalIA& g, int gi, bool energy);
-    bool grow_tiles();
+    bool grow_tiles(const std::vector<ListCtl>& ctl);
     uint32_t tile_lanes(const GlobalIA& g) const;
     void forces(double4* f, bool energy, int only, bool kick, bool advance = false);
     void launch_ul_accel(bool kick);
@@ -201,7 +208,7 @@ class Engine
     double* d_lpar_ = nullptr;
     double* d_tf_ = nullptr;
     double* d_te_ = nullptr;
-    uint32_t *d_gstart_ = nullptr, *d_gslot_ = nullptr;
+    uint32_t *d_gstart_ = nullptr, *d_tdst_ = nullptr;   // slots of each particle; slot of each term's body
     LocalSegTable segtab_{};
     uint32_t local_blocks_ = 0, n_slots_ = 0, n_terms_ = 0;
 
@@ -228,6 +235,11 @@ class Engine
     double* d_abs_margin_ = nullptr;
     int* d_never_ = nullptr;
     double* d_scratch_ = nullptr;   // N doubles
+    double4* d_noise_ = nullptr;    // the next step's draws (small systems)
+    bool small_ = false;            // k_forces evaluates the system and keeps its lists
+    bool tsp_ = false;              // has 3SPN2 terms
+    StepCtl* h_sctl_ = nullptr;     // pinned copies of the control words at a segment's end
+    ListCtl* h_lctl_ = nullptr;
     size_t scratch_n_ = 0;
 
     // graph of one step segment

@@ -1,9 +1,9 @@
 // Force kernels of the FP64 path.
 //
 // Local terms: one thread per term writes each body's force into its own slot of a term-force
-// buffer (no atomics); k_finish then sums, per particle, the slots that touch it in
-// interaction order and term order, i.e. in the order the reference's LocalForceField loop
-// accumulates them (LocalForceField.hpp:111-118).
+// buffer (no atomics); per particle the slots that touch it lie one after the other, in
+// interaction order and term order, and gather_force sums them in that order, i.e. in the order the
+// reference's LocalForceField loop accumulates them (LocalForceField.hpp:111-118).
 //
 // Pair terms: a group of lanes per participant walks its full (two-sided) list and reduces in
 // registers, so no atomics are needed and the sum order is fixed by the list.
@@ -29,7 +29,7 @@ struct LocalSeg
     uint32_t block_begin;   // first block of this segment in the launch
     uint32_t idx_off;       // into the flat index array
     uint32_t par_off;       // into the flat parameter array
-    uint32_t slot_off;      // first body slot (3 doubles per slot)
+    uint32_t slot_off;      // first body of the segment in the destination table
     uint32_t term_off;      // into the per-term energy array
 };
 constexpr int kMaxLocalSegs = 32;
@@ -39,19 +39,26 @@ struct LocalSegTable
     int n;
 };
 
-__device__ __forceinline__ void store3(double* f, uint32_t slot, double x, double y, double z)
+// Where a term's body forces go: dst[k] is the slot of the term's body k.
+struct TermOut
 {
-    f[3 * (size_t)slot + 0] = x; f[3 * (size_t)slot + 1] = y; f[3 * (size_t)slot + 2] = z;
+    double* f;
+    const uint32_t* dst;
+};
+__device__ __forceinline__ void store3(const TermOut& o, uint32_t body, double x, double y, double z)
+{
+    const size_t slot = 3 * (size_t)o.dst[body];
+    o.f[slot + 0] = x; o.f[slot + 1] = y; o.f[slot + 2] = z;
 }
 
-template<bool ENERGY>
-__device__ void local_term(const LocalSeg& s, uint32_t t, const double4* __restrict__ pos, const Box& box,
+template<bool ENERGY, bool TSP>
+__device__ __forceinline__ void local_term(const LocalSeg& s, uint32_t t, const double4* __restrict__ pos, const Box& box,
                            const uint32_t* __restrict__ idx, const double* __restrict__ par,
-                           double* __restrict__ tf, double* __restrict__ te)
+                           const uint32_t* __restrict__ dst, double* __restrict__ tfv, double* __restrict__ te)
 {
     const uint32_t* ix = idx + s.idx_off + (size_t)t * s.arity;
     const double* p = par + s.par_off + (size_t)t * s.npar;
-    const uint32_t slot = s.slot_off + t * s.nbody;
+    const TermOut tf{tfv, dst + s.slot_off + t * s.nbody};
     double energy = 0.0;
     if(s.kind == kBondHarmonic)
     {
@@ -65,8 +72,8 @@ __device__ void local_term(const LocalSeg& s, uint32_t t, const double4* __restr
         const double k = p[0], v0 = p[1];
         const double force = -1 * (2 * k * (len - v0));
         const double c = force * rlen;
-        store3(tf, slot + 0, -(dx * c), -(dy * c), -(dz * c));
-        store3(tf, slot + 1, dx * c, dy * c, dz * c);
+        store3(tf, 0, -(dx * c), -(dy * c), -(dz * c));
+        store3(tf, 1, dx * c, dy * c, dz * c);
         if(ENERGY) {const double dv = sqrt(len2) - v0; energy = k * dv * dv;}
     }
     else if(s.kind == kBondGo || s.kind == kContactGo)
@@ -100,8 +107,8 @@ __device__ void local_term(const LocalSeg& s, uint32_t t, const double4* __restr
                 energy = (v0 * 2.5 <= r) ? 0.0 : k * (5 * rd9 * rd3 - 6 * rd9 * rd);
             }
         }
-        store3(tf, slot + 0, -fx, -fy, -fz);
-        store3(tf, slot + 1, fx, fy, fz);
+        store3(tf, 0, -fx, -fy, -fz);
+        store3(tf, 1, fx, fy, fz);
     }
     else if(s.kind == kAngleHarmonic || s.kind == kAngleGaussian)
     {
@@ -138,9 +145,9 @@ __device__ void local_term(const LocalSeg& s, uint32_t t, const double4* __restr
         const double ci = cis * inv_ij, ck = cis * inv_kj;
         const double Fix = ci * (cos_theta * eix - ekx), Fiy = ci * (cos_theta * eiy - eky), Fiz = ci * (cos_theta * eiz - ekz);
         const double Fkx = ck * (cos_theta * ekx - eix), Fky = ck * (cos_theta * eky - eiy), Fkz = ck * (cos_theta * ekz - eiz);
-        store3(tf, slot + 0, Fix, Fiy, Fiz);
-        store3(tf, slot + 1, -Fix - Fkx, -Fiy - Fky, -Fiz - Fkz);
-        store3(tf, slot + 2, Fkx, Fky, Fkz);
+        store3(tf, 0, Fix, Fiy, Fiz);
+        store3(tf, 1, -Fix - Fkx, -Fiy - Fky, -Fiz - Fkz);
+        store3(tf, 2, Fkx, Fky, Fkz);
         energy = pot;
     }
     else if(s.kind == kDihedralClementi)
@@ -179,13 +186,14 @@ __device__ void local_term(const LocalSeg& s, uint32_t t, const double4* __restr
         const double Flx = cl * nx, Fly = cl * ny, Flz = cl * nz;
         const double coef_ijk = (ijx * kjx + ijy * kjy + ijz * kjz) * r_kj_rlensq;
         const double coef_jkl = (klx * kjx + kly * kjy + klz * kjz) * r_kj_rlensq;
-        store3(tf, slot + 0, Fix, Fiy, Fiz);
-        store3(tf, slot + 1, (coef_ijk - 1.0) * Fix - coef_jkl * Flx, (coef_ijk - 1.0) * Fiy - coef_jkl * Fly,
+        store3(tf, 0, Fix, Fiy, Fiz);
+        store3(tf, 1, (coef_ijk - 1.0) * Fix - coef_jkl * Flx, (coef_ijk - 1.0) * Fiy - coef_jkl * Fly,
                (coef_ijk - 1.0) * Fiz - coef_jkl * Flz);
-        store3(tf, slot + 2, (coef_jkl - 1.0) * Flx - coef_ijk * Fix, (coef_jkl - 1.0) * Fly - coef_ijk * Fiy,
+        store3(tf, 2, (coef_jkl - 1.0) * Flx - coef_ijk * Fix, (coef_jkl - 1.0) * Fly - coef_ijk * Fiy,
                (coef_jkl - 1.0) * Flz - coef_ijk * Fiz);
-        store3(tf, slot + 3, Flx, Fly, Flz);
+        store3(tf, 3, Flx, Fly, Flz);
     }
+    else if(!TSP) {}
     else if(s.kind == kBond3SPN2)
     {
         // BondLengthInteraction.hpp:126-148; ThreeSPN2BondPotential.hpp:22-35
@@ -199,8 +207,8 @@ __device__ void local_term(const LocalSeg& s, uint32_t t, const double4* __restr
         const double dv = len - v0;
         const double force = -1 * (2 * k * (dv + 200 * dv * dv * dv));
         const double c = force * rlen;
-        store3(tf, slot + 0, -(dx * c), -(dy * c), -(dz * c));
-        store3(tf, slot + 1, dx * c, dy * c, dz * c);
+        store3(tf, 0, -(dx * c), -(dy * c), -(dz * c));
+        store3(tf, 1, dx * c, dy * c, dz * c);
         if(ENERGY) {const double ev = sqrt(len2) - v0; const double ev2 = ev * ev; energy = k * (ev2 + 100 * ev2 * ev2);}
     }
     else if(s.kind == kDihedralPGauss)
@@ -235,12 +243,12 @@ __device__ void local_term(const LocalSeg& s, uint32_t t, const double4* __restr
         const double Flx = cl * nx, Fly = cl * ny, Flz = cl * nz;
         const double coef_ijk = (ijx * kjx + ijy * kjy + ijz * kjz) * r_kj_rlensq;
         const double coef_jkl = (klx * kjx + kly * kjy + klz * kjz) * r_kj_rlensq;
-        store3(tf, slot + 0, Fix, Fiy, Fiz);
-        store3(tf, slot + 1, (coef_ijk - 1.0) * Fix - coef_jkl * Flx, (coef_ijk - 1.0) * Fiy - coef_jkl * Fly,
+        store3(tf, 0, Fix, Fiy, Fiz);
+        store3(tf, 1, (coef_ijk - 1.0) * Fix - coef_jkl * Flx, (coef_ijk - 1.0) * Fiy - coef_jkl * Fly,
                (coef_ijk - 1.0) * Fiz - coef_jkl * Flz);
-        store3(tf, slot + 2, (coef_jkl - 1.0) * Flx - coef_ijk * Fix, (coef_jkl - 1.0) * Fly - coef_ijk * Fiy,
+        store3(tf, 2, (coef_jkl - 1.0) * Flx - coef_ijk * Fix, (coef_jkl - 1.0) * Fly - coef_ijk * Fiy,
                (coef_jkl - 1.0) * Flz - coef_ijk * Fiz);
-        store3(tf, slot + 3, Flx, Fly, Flz);
+        store3(tf, 3, Flx, Fly, Flz);
     }
     else if(s.kind == kBaseStacking)
     {
@@ -249,9 +257,9 @@ __device__ void local_term(const LocalSeg& s, uint32_t t, const double4* __restr
         const tsp::GlobalPos acc{pos, box};
         tsp::V3<double> fSi, fBi, fBj;
         const double en = tsp::base_stack<double, ENERGY>(ix[0], ix[1], ix[2], (int)p[0], acc, fSi, fBi, fBj);
-        store3(tf, slot + 0, fSi.x, fSi.y, fSi.z);
-        store3(tf, slot + 1, fBi.x, fBi.y, fBi.z);
-        store3(tf, slot + 2, fBj.x, fBj.y, fBj.z);
+        store3(tf, 0, fSi.x, fSi.y, fSi.z);
+        store3(tf, 1, fBi.x, fBi.y, fBi.z);
+        store3(tf, 2, fBj.x, fBj.y, fBj.z);
         if(ENERGY) {energy = en;}
     }
     if(ENERGY) {te[s.term_off + t] = energy;}
@@ -262,7 +270,7 @@ __device__ void local_term(const LocalSeg& s, uint32_t t, const double4* __restr
 template<bool ENERGY>
 __global__ void __launch_bounds__(256)
 k_local_terms(const double4* __restrict__ pos, Box box, LocalSegTable tab,
-              const uint32_t* __restrict__ idx, const double* __restrict__ par,
+              const uint32_t* __restrict__ idx, const double* __restrict__ par, const uint32_t* __restrict__ dst,
               double* __restrict__ tf, double* __restrict__ te, int only_seg)
 {
     int si = 0;
@@ -271,7 +279,7 @@ k_local_terms(const double4* __restrict__ pos, Box box, LocalSegTable tab,
     const LocalSeg s = tab.seg[si];
     const uint32_t t = (blockIdx.x - s.block_begin) * blockDim.x + threadIdx.x;
     if(t >= s.n_terms) {return;}
-    local_term<ENERGY>(s, t, pos, box, idx, par, tf, te);
+    local_term<ENERGY, true>(s, t, pos, box, idx, par, dst, tf, te);
 }
 
 struct PairParams
@@ -293,6 +301,19 @@ template<int NPAR> struct GlobalPar
     __device__ __forceinline__ double get(uint32_t key, int c) const {return p[(size_t)NPAR * key + c];}
 };
 template<int KIND> constexpr int pair_npar() {return KIND == kPairLJ ? 2 : 1;}
+// the parameters of one pair in registers: key 0 the owner, key 1 the partner
+struct RegPar
+{
+    double a0, a1, b0, b1;
+    __device__ __forceinline__ double get(uint32_t key, int c) const {return key ? (c ? b1 : b0) : (c ? a1 : a0);}
+};
+template<int KIND> __device__ __forceinline__ void load_par(const double* __restrict__ ppar, uint32_t i, double& p0,
+                                                            double& p1)
+{
+    constexpr int N = pair_npar<KIND>();
+    p0 = ppar[(size_t)N * i];
+    p1 = (N > 1) ? ppar[(size_t)N * i + 1] : 0.0;
+}
 
 // Pair force on the owner i from j (full list).  d = adjust_direction(r_i, r_j).  i and j are
 // particle indices (the energy of a pair is counted from its lower particle, and the
@@ -375,14 +396,6 @@ __device__ __forceinline__ void pair_term_p(const PairParams& pp, uint32_t i, ui
     }
 }
 
-template<int KIND, bool ENERGY>
-__device__ __forceinline__ void pair_term(const PairParams& pp, uint32_t i, uint32_t j, const double* __restrict__ ppar,
-                                          double dx, double dy, double dz,
-                                          double& fx, double& fy, double& fz, double& e)
-{
-    pair_term_p<KIND, ENERGY>(pp, i, j, GlobalPar<pair_npar<KIND>()>{ppar}, i, j, dx, dy, dz, fx, fy, fz, e);
-}
-
 // ------------------------------------------------------------------------------------
 // Pair forces, fused over every global interaction: blocks are split into one segment per
 // interaction; inside a segment `tpp` lanes share one participant (sorted slot t), split its
@@ -394,8 +407,7 @@ struct PairSeg
 {
     int kind;
     uint32_t tpp, np, block_begin, cap;
-    const uint32_t* part;
-    const uint32_t* order;
+    const uint32_t* spart;   // particle of each sorted slot
     const uint32_t* nl;
     const uint32_t* nn;
     const double* ppar;
@@ -411,23 +423,29 @@ struct PairSegTable
 };
 
 // A lane's entries of a row, kPairBatch at a time: the list words and then the partners'
-// positions of a batch are all in flight before the first pair is computed (one dependent load
-// pair per entry would leave the lane waiting on memory); the lane still takes its entries
-// k = l, l + tpp, ... in increasing order, so its sum order is the unbatched one.
+// positions and parameters of a batch are all in flight before the first pair is computed (one
+// dependent load per entry would leave the lane waiting on memory); the lane still takes its
+// entries k = l, l + tpp, ... in increasing order, so its sum order is the unbatched one.  A row's
+// chain of dependent loads is its length, particle and list words, then positions and parameters:
+// at a few thousand particles each level is a miss to memory of 0.5 to 1 us, and the kernel is
+// little else.
 constexpr int kPairBatch = 4;
 
 template<int KIND, bool ENERGY>
 __device__ __forceinline__ void pair_row(const PairSeg& s, uint32_t t, uint32_t l, const double4* __restrict__ pos,
                                          const Box& box, double& fx, double& fy, double& fz, double& e, uint32_t& i)
 {
-    i = s.part[s.order[t]];
-    const double4 ri = pos[i];
+    i = s.spart[t];
     const uint32_t cnt = s.nn[t];
     const uint32_t* row = s.nl + (size_t)t * s.cap;
+    const double4 ri = pos[i];
+    RegPar par;
+    load_par<KIND>(s.ppar, i, par.a0, par.a1);
     for(uint32_t k0 = l; k0 < cnt; k0 += kPairBatch * s.tpp)
     {
         uint32_t j[kPairBatch];
         double4 rj[kPairBatch];
+        double p0[kPairBatch], p1[kPairBatch];
 #pragma unroll
         for(int m = 0; m < kPairBatch; ++m)
         {
@@ -435,28 +453,24 @@ __device__ __forceinline__ void pair_row(const PairSeg& s, uint32_t t, uint32_t 
             j[m] = (k < cnt) ? row[k] : i;
         }
 #pragma unroll
-        for(int m = 0; m < kPairBatch; ++m) {rj[m] = pos[j[m]];}
+        for(int m = 0; m < kPairBatch; ++m) {rj[m] = pos[j[m]]; load_par<KIND>(s.ppar, j[m], p0[m], p1[m]);}
 #pragma unroll
         for(int m = 0; m < kPairBatch; ++m)
         {
             if(k0 + m * s.tpp >= cnt) {break;}
             double dx, dy, dz;
             adjust_direction(box, ri.x, ri.y, ri.z, rj[m].x, rj[m].y, rj[m].z, dx, dy, dz);
-            pair_term<KIND, ENERGY>(s.pp, i, j[m], s.ppar, dx, dy, dz, fx, fy, fz, e);
+            par.b0 = p0[m]; par.b1 = p1[m];
+            pair_term_p<KIND, ENERGY>(s.pp, i, j[m], par, 0, 1, dx, dy, dz, fx, fy, fz, e);
         }
     }
 }
 
+// one row by the tpp lanes of a group: its force (and energy) stored by lane 0
 template<bool ENERGY>
-__global__ void __launch_bounds__(256)
-k_pairs(const double4* __restrict__ pos, Box box, PairSegTable tab)
+__device__ __forceinline__ void pair_row_store(const PairSeg& s, uint32_t t, uint32_t l, const double4* __restrict__ pos,
+                                               const Box& box)
 {
-    int si = 0;
-    while(si + 1 < tab.n && blockIdx.x >= tab.seg[si + 1].block_begin) {++si;}
-    const PairSeg& s = tab.seg[si];
-    const uint32_t gt = (blockIdx.x - s.block_begin) * blockDim.x + threadIdx.x;
-    const uint32_t t = gt / s.tpp, l = gt % s.tpp;
-    if(t >= s.np) {return;}   // whole groups leave together
     double fx = 0, fy = 0, fz = 0, e = 0;
     uint32_t i = 0;
     if(s.kind == kPairLJ) {pair_row<kPairLJ, ENERGY>(s, t, l, pos, box, fx, fy, fz, e, i);}
@@ -475,6 +489,19 @@ k_pairs(const double4* __restrict__ pos, Box box, PairSegTable tab)
         s.fout[i] = make_double4(fx, fy, fz, 0.0);
         if(ENERGY) {s.eout[t] = e;}
     }
+}
+
+template<bool ENERGY>
+__global__ void __launch_bounds__(256)
+k_pairs(const double4* __restrict__ pos, Box box, PairSegTable tab)
+{
+    int si = 0;
+    while(si + 1 < tab.n && blockIdx.x >= tab.seg[si + 1].block_begin) {++si;}
+    const PairSeg& s = tab.seg[si];
+    const uint32_t gt = (blockIdx.x - s.block_begin) * blockDim.x + threadIdx.x;
+    const uint32_t t = gt / s.tpp, l = gt % s.tpp;
+    if(t >= s.np) {return;}   // whole groups leave together
+    pair_row_store<ENERGY>(s, t, l, pos, box);
 }
 
 // ------------------------------------------------------------------------------------
@@ -570,14 +597,17 @@ __device__ __forceinline__ void pair_row_mixed(const PairSeg& s, uint32_t t, uin
                                                uint32_t& i)
 {
     const PairConstsF K = pair_consts_f(s.pp);
-    i = s.part[s.order[t]];
-    const double4 ri = pos[i];
+    i = s.spart[t];
     const uint32_t cnt = s.nn[t];
     const uint32_t* row = s.nl + (size_t)t * s.cap;
+    const double4 ri = pos[i];
+    RegPar par;
+    load_par<KIND>(s.ppar, i, par.a0, par.a1);
     for(uint32_t k0 = l; k0 < cnt; k0 += kPairBatch * s.tpp)
     {
         uint32_t j[kPairBatch];
         double4 rj[kPairBatch];
+        double p0[kPairBatch], p1[kPairBatch];
 #pragma unroll
         for(int m = 0; m < kPairBatch; ++m)
         {
@@ -585,19 +615,16 @@ __device__ __forceinline__ void pair_row_mixed(const PairSeg& s, uint32_t t, uin
             j[m] = (k < cnt) ? row[k] : i;
         }
 #pragma unroll
-        for(int m = 0; m < kPairBatch; ++m) {rj[m] = pos[j[m]];}
+        for(int m = 0; m < kPairBatch; ++m) {rj[m] = pos[j[m]]; load_par<KIND>(s.ppar, j[m], p0[m], p1[m]);}
 #pragma unroll
         for(int m = 0; m < kPairBatch; ++m)
         {
             if(k0 + m * s.tpp >= cnt) {break;}
             double ddx, ddy, ddz;
             adjust_direction(box, ri.x, ri.y, ri.z, rj[m].x, rj[m].y, rj[m].z, ddx, ddy, ddz);
+            par.b0 = p0[m]; par.b1 = p1[m];
             float c;
-            if(!pair_term_f32<KIND, ENERGY>(K, s.pp, GlobalPar<pair_npar<KIND>()>{s.ppar}, i, j[m], i, j[m], ddx, ddy,
-                                            ddz, c, e))
-            {
-                continue;
-            }
+            if(!pair_term_f32<KIND, ENERGY>(K, s.pp, par, i, j[m], 0, 1, ddx, ddy, ddz, c, e)) {continue;}
             const float dx = (float)ddx, dy = (float)ddy, dz = (float)ddz;
             long long fx, fy, fz;
             fix3r<float>(dx * c, dy * c, dz * c, fx, fy, fz);
@@ -613,15 +640,9 @@ __device__ __forceinline__ long long shfl_xor_ll(long long v, int o)
 }
 
 template<bool ENERGY>
-__global__ void __launch_bounds__(256)
-k_pairs_mixed(const double4* __restrict__ pos, Box box, PairSegTable tab)
+__device__ __forceinline__ void pair_row_mixed_store(const PairSeg& s, uint32_t t, uint32_t l,
+                                                     const double4* __restrict__ pos, const Box& box)
 {
-    int si = 0;
-    while(si + 1 < tab.n && blockIdx.x >= tab.seg[si + 1].block_begin) {++si;}
-    const PairSeg& s = tab.seg[si];
-    const uint32_t gt = (blockIdx.x - s.block_begin) * blockDim.x + threadIdx.x;
-    const uint32_t t = gt / s.tpp, l = gt % s.tpp;
-    if(t >= s.np) {return;}   // whole groups leave together
     long long ax = 0, ay = 0, az = 0;
     double e = 0;
     uint32_t i = 0;
@@ -647,18 +668,81 @@ k_pairs_mixed(const double4* __restrict__ pos, Box box, PairSegTable tab)
     }
 }
 
-// Per particle: the local-term slots (in interaction, term order) plus every pair
-// interaction's force; stores the force and, with kick != 0, applies the velocity half-kick
+template<bool ENERGY>
+__global__ void __launch_bounds__(256)
+k_pairs_mixed(const double4* __restrict__ pos, Box box, PairSegTable tab)
+{
+    int si = 0;
+    while(si + 1 < tab.n && blockIdx.x >= tab.seg[si + 1].block_begin) {++si;}
+    const PairSeg& s = tab.seg[si];
+    const uint32_t gt = (blockIdx.x - s.block_begin) * blockDim.x + threadIdx.x;
+    const uint32_t t = gt / s.tpp, l = gt % s.tpp;
+    if(t >= s.np) {return;}   // whole groups leave together
+    pair_row_mixed_store<ENERGY>(s, t, l, pos, box);
+}
+
+// The force on one particle: its local-term slots (in interaction, term order) plus every pair
+// interaction's force in interaction order.  A 3SPN2 multibody interaction is read from its
+// fixed-point sums where fg[g] is null (acc[g], the flag word after them).
+struct GatherArgs
+{
+    const uint32_t* gstart;            // null: no local terms
+    const double* tf;
+    const double4* fg[kMaxPairSegs];
+    unsigned long long* acc[kMaxPairSegs];
+    int ng;
+};
+template<bool CLEAR>
+__device__ __forceinline__ void gather_force(const GatherArgs& a, uint32_t n, uint32_t i, double& x, double& y, double& z)
+{
+    x = 0; y = 0; z = 0;
+    if(a.gstart != nullptr)
+    {
+        // four slots' loads in flight at a time, added in order
+        const uint32_t b = a.gstart[i], e = a.gstart[i + 1];
+        for(uint32_t k = b; k < e; k += 4)
+        {
+            double v[12];
+#pragma unroll
+            for(uint32_t q = 0; q < 4; ++q)
+            {
+                const uint32_t s = (k + q < e) ? k + q : b;
+#pragma unroll
+                for(int c = 0; c < 3; ++c) {v[3 * q + c] = a.tf[3 * (size_t)s + c];}
+            }
+#pragma unroll
+            for(uint32_t q = 0; q < 4; ++q)
+            {
+                if(k + q < e) {x += v[3 * q]; y += v[3 * q + 1]; z += v[3 * q + 2];}
+            }
+        }
+    }
+    for(int g = 0; g < a.ng; ++g)
+    {
+        if(a.fg[g] != nullptr)
+        {
+            const double4 f = a.fg[g][i];
+            x += f.x; y += f.y; z += f.z;
+        }
+        else
+        {
+            unsigned long long* s = a.acc[g] + 3 * (size_t)i;
+            const double bad = a.acc[g][3 * (size_t)n] ? __builtin_nan("") : 0.0;
+            x += (double)(long long)s[0] * tsp::kFixInv + bad;
+            y += (double)(long long)s[1] * tsp::kFixInv + bad;
+            z += (double)(long long)s[2] * tsp::kFixInv + bad;
+            if(CLEAR) {s[0] = 0ull; s[1] = 0ull; s[2] = 0ull;}
+        }
+    }
+}
+
+// Stores the force of every particle and, with kick != 0, applies the velocity half-kick
 // v += (dt/2) (1/m) f of BAOAB (BAOABLangevinIntegrator.hpp:222-229) and G-JF
 // (GJFNVTLangevinIntegrator.hpp:222-229, (dt 0.5) rm == (dt/2) rm); with advance != 0 it advances
 // the step count.
 struct FinishArgs
 {
-    const uint32_t* gstart;
-    const uint32_t* gslot;
-    const double* tf;
-    const double4* fg[kMaxPairSegs];
-    int ng;
+    GatherArgs g;
     double halfdt;
     int kick;       // apply the half-kick
     int advance;    // advance the step count (set with kick, or alone)
@@ -671,21 +755,8 @@ k_finish(uint32_t n, FinishArgs a, double4* __restrict__ force, double4* __restr
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if(i < n)
     {
-        double x = 0, y = 0, z = 0;
-        if(a.gstart != nullptr)
-        {
-            const uint32_t b = a.gstart[i], e = a.gstart[i + 1];
-            for(uint32_t k = b; k < e; ++k)
-            {
-                const uint32_t sl = a.gslot[k];
-                x += a.tf[3 * (size_t)sl + 0]; y += a.tf[3 * (size_t)sl + 1]; z += a.tf[3 * (size_t)sl + 2];
-            }
-        }
-        for(int g = 0; g < a.ng; ++g)
-        {
-            const double4 f = a.fg[g][i];
-            x += f.x; y += f.y; z += f.z;
-        }
+        double x, y, z;
+        gather_force<false>(a.g, n, i, x, y, z);
         force[i] = make_double4(x, y, z, 0.0);
         if(a.kick)
         {

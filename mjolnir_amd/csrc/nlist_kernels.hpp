@@ -351,7 +351,6 @@ struct ListSeg
     uint32_t* nl;
     uint16_t* nl16;                    // non-null: also the staging slot of each entry (k_pairs_tiled)
     uint32_t* nn;
-    uint32_t* order;
     uint32_t* spart;                   // particle of each sorted slot
     const double4* spos;               // its position at this build (cell lists)
     ListCtl* ctl;
@@ -454,7 +453,7 @@ __device__ __forceinline__ void verlet_row(const ListSeg& s, uint32_t t, uint32_
     uint32_t p, i;
     if(s.allpairs) {p = t;} else {p = s.svals[t];}
     i = s.part[p];
-    if(l == 0) {s.order[t] = p; s.spart[t] = i;}
+    if(l == 0) {s.spart[t] = i;}
     RowBuild rb;
     rb.i = i;
     rb.ri = pos[i];
@@ -607,7 +606,7 @@ __device__ __forceinline__ int margin_decision(ListCtl& c, double dmargin, doubl
 }
 
 __global__ void __launch_bounds__(1024)
-k_prep_small(const double4* __restrict__ pos, PrepSegTable tab, StepCtl* __restrict__ sctl, int force)
+k_prep_small(const double4* __restrict__ pos, PrepSegTable tab, StepCtl* __restrict__ sctl, uint32_t k, int force)
 {
     __shared__ uint32_t key[kSmallMaxPart];
     __shared__ uint32_t sval[kSmallMaxPart];
@@ -620,7 +619,7 @@ k_prep_small(const double4* __restrict__ pos, PrepSegTable tab, StepCtl* __restr
     const uint32_t tid = threadIdx.x, nt = blockDim.x;
     if(tid == 0)
     {
-        const double dmargin = 2 * sqrt(__longlong_as_double((long long)sctl->maxdisp2[sctl->step & 1]));
+        const double dmargin = 2 * sqrt(__longlong_as_double((long long)sctl->maxdisp2[(sctl->step + k) & 1]));
         go = margin_decision(*s.ctl, dmargin, s.abs_margin, s.never_rebuild, force);
         if(go) {atomicAdd(&sctl->rebuilds, 1ull);}
     }
@@ -735,13 +734,14 @@ k_prep_small(const double4* __restrict__ pos, PrepSegTable tab, StepCtl* __restr
 }
 
 // Skin check for interactions on the multi-kernel (counting-sort) path.
-__global__ void k_margin_large(PrepSegTable tab, StepCtl* __restrict__ sctl, int force)
+// k: the step's number since StepCtl::step was last advanced
+__global__ void k_margin_large(PrepSegTable tab, StepCtl* __restrict__ sctl, uint32_t k, int force)
 {
     const int g = threadIdx.x;
     if(g < tab.n)
     {
         const PrepSeg& s = tab.seg[g];
-        const double dmargin = 2 * sqrt(__longlong_as_double((long long)sctl->maxdisp2[sctl->step & 1]));
+        const double dmargin = 2 * sqrt(__longlong_as_double((long long)sctl->maxdisp2[(sctl->step + k) & 1]));
         if(margin_decision(*s.ctl, dmargin, s.abs_margin, s.never_rebuild, force)) {atomicAdd(&sctl->rebuilds, 1ull);}
     }
 }

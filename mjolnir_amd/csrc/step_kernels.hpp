@@ -1,0 +1,331 @@
+// The two kernels of an integrator step inside a segment of steps.
+//
+// k_advance closes one step and opens the next: the forces summed per particle, the closing
+// half-kick, the next step's position update and its largest displacement.  One pass over the
+// state instead of two (k_finish and k_baoab_a / k_gjf_a), with no force array written in between:
+// 184 instead of 320 bytes a particle for a Lennard-Jones fluid.
+//
+// k_forces evaluates every interaction of a small system in one launch, its blocks split into one
+// run per interaction, and keeps the neighbour lists: every block takes the step's skin decision
+// for itself from the same two words, and on a rebuild each row group first finds its own row
+// among all participants.  A step of a small system is a chain of dependent launches, each about
+// 1 us of dispatch plus two or three levels of loads that miss to memory (0.5 to 1 us each), so
+// what counts is their number: two here, where separate kernels for the skin check, the cell sort,
+// the list build, the local terms, the pairs, each 3SPN2 interaction, the force sum and the
+// position update make 6 (a fluid) to 17 (a DNA duplex).  A rebuild by brute force is np^2 distance
+// tests without any ordering between blocks: 75 us at 4096 participants, where the cell sort and
+// the build from it took 180.  Measured per FP64 step, before and after: a fluid of 512 particles
+// 17.0 -> 9.4 us, of 4096 19.1 -> 11.4, a chain of 1000 beads 29.3 -> 12.5, a 200-bp duplex
+// 66 -> 28; mixed chain of 3001 beads 33 -> 14.5.
+#pragma once
+#include "force_kernels.hpp"
+#include "nlist_kernels.hpp"
+
+namespace mjg
+{
+// the lists that k_forces keeps: their margins are settled by the next k_advance
+constexpr int kMaxSelfLists = 4;
+struct SelfLists
+{
+    ListCtl* ctl[kMaxSelfLists];
+    double abs_margin[kMaxSelfLists];
+    int never[kMaxSelfLists];          // Naive: built once
+    int n;
+};
+
+// The skin decision of step k of the segment (ForceField::reduce_margin, ForceField.hpp:75-92): the
+// margin left after the step's largest displacement, below zero when the list must be rebuilt.
+__device__ __forceinline__ double margin_after(const ListCtl* ctl, const StepCtl* sctl, uint32_t k)
+{
+    return ctl->margin - 2 * sqrt(__longlong_as_double((long long)sctl->maxdisp2[(sctl->step + k) & 1]));
+}
+
+struct AdvanceArgs
+{
+    GatherArgs g;
+    SelfLists lists;
+    double4* pos;
+    double4* vel;
+    double4* force;
+    const double* rmass;
+    const double* c1;
+    const double* c2;
+    const double* c3;
+    const double4* noise;      // the step's draws where k_forces made them (null: drawn here)
+    StepCtl* ctl;
+    const ListCtl* lctl;       // every list's control words
+    ListCtl* h_lctl;           // their pinned copy, and that of the step control, for the host
+    StepCtl* h_ctl;
+    double dt, halfdt;
+    uint64_t seed;
+    Box box;
+    uint32_t n;
+    uint32_t k;                // steps since the segment began (ctl->step does not move inside it)
+    int nlists;
+};
+
+// FIRST: opens step 0 from the stored force.  LAST: closes step k - 1 only, stores the force,
+// advances the step count by k and reports to the host.
+template<bool GJF, bool FIRST, bool LAST>
+__global__ void __launch_bounds__(256)
+k_advance(AdvanceArgs a)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t step0 = a.ctl->step;
+    if constexpr(!FIRST)
+    {
+        // the previous step's skin decision, taken by every block of its k_forces, is made final
+        if(blockIdx.x == 0 && threadIdx.x < (uint32_t)kWave)
+        {
+            bool spent = false;
+            if(threadIdx.x < (uint32_t)a.lists.n && !a.lists.never[threadIdx.x])
+            {
+                ListCtl* c = a.lists.ctl[threadIdx.x];
+                const double m = margin_after(c, a.ctl, a.k - 1);
+                spent = m < 0;
+                c->margin = spent ? a.lists.abs_margin[threadIdx.x] : m;
+            }
+            const uint32_t built = (uint32_t)__popcll(__ballot(spent));
+            if(threadIdx.x == 0 && built > 0) {a.ctl->rebuilds += built;}
+        }
+    }
+    double d2 = 0.0;
+    if(i < a.n)
+    {
+        double fx, fy, fz;
+        const double rm = a.rmass[i];
+        double4 v = a.vel[i];
+        double4 p;
+        if constexpr(!LAST) {p = a.pos[i];}
+        double Rx = 0, Ry = 0, Rz = 0;
+        double b = 0, c = 0, cc = 0;
+        if constexpr(!LAST)
+        {
+            b = a.c1[i]; c = a.c2[i];
+            if constexpr(GJF) {cc = a.c3[i];}
+            if(!FIRST && a.noise) {const double4 r = a.noise[i]; Rx = r.x; Ry = r.y; Rz = r.z;}
+            else {noise3(a.seed, step0 + a.k, i, Rx, Ry, Rz);}
+        }
+        if constexpr(FIRST) {const double4 f = a.force[i]; fx = f.x; fy = f.y; fz = f.z;}
+        else
+        {
+            gather_force<true>(a.g, a.n, i, fx, fy, fz);
+            // closing half-kick (BAOABLangevinIntegrator.hpp:222-229, GJFNVTLangevinIntegrator.hpp:222-229)
+            const double hrm = a.halfdt * rm;
+            v.x += hrm * fx; v.y += hrm * fy; v.z += hrm * fz;
+        }
+        if constexpr(LAST) {a.force[i] = make_double4(fx, fy, fz, 0.0);}
+        else
+        {
+            double dpx, dpy, dpz;
+            if constexpr(!GJF)
+            {
+                // BAOABLangevinIntegrator.hpp:176-200
+                const double hrm = a.halfdt * rm;
+                v.x += hrm * fx; v.y += hrm * fy; v.z += hrm * fz;
+                dpx = a.halfdt * v.x; dpy = a.halfdt * v.y; dpz = a.halfdt * v.z;
+                v.x *= b; v.y *= b; v.z *= b;
+                v.x += c * Rx; v.y += c * Ry; v.z += c * Rz;
+                dpx += a.halfdt * v.x; dpy += a.halfdt * v.y; dpz += a.halfdt * v.z;
+            }
+            else
+            {
+                // GJFNVTLangevinIntegrator.hpp:172-197
+                const double r2m = 0.5 * rm;
+                const double bx = Rx * c, by = Ry * c, bz = Rz * c;
+                const double bdt = b * a.dt;
+                dpx = bdt * (v.x + r2m * (a.dt * fx + bx));
+                dpy = bdt * (v.y + r2m * (a.dt * fy + by));
+                dpz = bdt * (v.z + r2m * (a.dt * fz + bz));
+                const double dtr2m = a.dt * r2m, brm = b * rm;
+                v.x = cc * (v.x + dtr2m * fx) + brm * bx;
+                v.y = cc * (v.y + dtr2m * fy) + brm * by;
+                v.z = cc * (v.z + dtr2m * fz) + brm * bz;
+            }
+            double x = p.x + dpx, y = p.y + dpy, z = p.z + dpz;
+            adjust_position(a.box, x, y, z);
+            p.x = x; p.y = y; p.z = z;
+            a.pos[i] = p;
+            d2 = length_sq(dpx, dpy, dpz);
+            if(!isfinite(x) || !isfinite(y) || !isfinite(z)) {a.ctl->nonfinite = 1;}
+        }
+        a.vel[i] = v;
+    }
+    if constexpr(!LAST) {block_max_to(d2, a.ctl, step0 + a.k);}
+    else if(blockIdx.x == 0)
+    {
+        // every other kernel of the segment has ended: the control words are final after this
+        __syncthreads();
+        if(threadIdx.x == 0)
+        {
+            StepCtl c = *a.ctl;
+            c.step += a.k;
+            a.ctl->step = c.step;
+            *a.h_ctl = c;
+        }
+        if(threadIdx.x < (uint32_t)a.nlists) {a.h_lctl[threadIdx.x] = a.lctl[threadIdx.x];}
+    }
+}
+
+// The segment's start, from which a segment whose list overflowed runs again.
+struct BackupArgs
+{
+    const double4* src[3];
+    double4* dst[3];
+    const StepCtl* ctl;
+    StepCtl* bak_ctl;
+    const ListCtl* lctl;
+    ListCtl* bak_lctl;
+    uint32_t n;
+    int nlists;
+};
+__global__ void __launch_bounds__(256)
+k_backup(BackupArgs a)
+{
+    for(uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x)
+    {
+#pragma unroll
+        for(int k = 0; k < 3; ++k) {a.dst[k][i] = a.src[k][i];}
+    }
+    if(blockIdx.x == 0)
+    {
+        if(threadIdx.x == 0) {*a.bak_ctl = *a.ctl;}
+        if(threadIdx.x < (uint32_t)a.nlists) {a.bak_lctl[threadIdx.x] = a.lctl[threadIdx.x];}
+    }
+}
+
+// ------------------------------------------------------------------------------------
+// all forces of a small system
+// ------------------------------------------------------------------------------------
+constexpr int kMaxSmallLocals = 8;
+constexpr int kSmallSeg = 8;         // blocks' runs: global interactions, local terms, noise
+
+// one global interaction: its rows and what keeps its list
+struct RowSeg
+{
+    uint32_t block_begin;
+    int never;
+    PairSeg p;                 // LJ / EV / DH / 3SPN2 excluded volume
+    unsigned long long* acc;   // 3SPN2 multibody: fixed-point sums
+    ListCtl* ctl;
+    uint32_t* nl;
+    uint32_t* nn;
+    const uint32_t* part;
+    const uint32_t* pslot;
+    const uint32_t* mol;
+    const uint32_t* ex_start;
+    const uint32_t* ex;
+    ListRule rule;
+};
+struct SmallForces
+{
+    RowSeg row[kMaxSelfLists];
+    LocalSeg local[kMaxSmallLocals];
+    int nrow, nlocal;
+    uint32_t local_begin, noise_begin;   // first blocks of the local terms and of the noise
+    const uint32_t* lidx;
+    const double* lpar;
+    const uint32_t* ldst;
+    double* tf;
+    double4* noise;
+    uint64_t seed;
+    StepCtl* sctl;
+    uint32_t n, k;
+};
+constexpr uint32_t kScanTile = 256;   // candidates staged at a time by a rebuild
+
+// The rows of one block found among all participants, in participant order (the pairs and the test
+// are k_verlet's).  Every thread of the block calls it; `valid`: the thread's row exists.
+__device__ __forceinline__ void self_build(const RowSeg& s, const Box& box, const double4* __restrict__ pos, uint32_t t,
+                                           uint32_t l, bool valid)
+{
+    __shared__ double cx[kScanTile], cy[kScanTile], cz[kScanTile];
+    __shared__ uint32_t cj[kScanTile];
+    const uint32_t tid = threadIdx.x, lane = tid % kWave;
+    const uint32_t np = s.p.np, tpp = s.p.tpp;
+    ListSeg ls{};
+    ls.cap = s.p.cap;
+    ls.pslot = s.pslot; ls.mol = s.mol; ls.ex_start = s.ex_start; ls.ex = s.ex;
+    ls.rule = s.rule;
+    RowBuild rb;
+    rb.i = valid ? s.p.spart[t] : 0u;
+    rb.ri = pos[rb.i];
+    rb.gmask = group_mask_of(tpp, lane);
+    rb.below = rb.gmask & ((1ull << lane) - 1ull);
+    rb.count = 0;
+    rb.row = s.nl + (size_t)(valid ? t : 0u) * s.p.cap;
+    rb.row16 = nullptr;
+    for(uint32_t base = 0; base < np; base += kScanTile)
+    {
+        const uint32_t q = base + tid;
+        if(q < np)
+        {
+            const uint32_t j = s.part[q];
+            const double4 r = pos[j];
+            cx[tid] = r.x; cy[tid] = r.y; cz[tid] = r.z; cj[tid] = j;
+        }
+        __syncthreads();
+        const uint32_t m = (np - base < kScanTile) ? np - base : kScanTile;
+        for(uint32_t b = 0; b < m; b += tpp)
+        {
+            const uint32_t c = b + l;
+            const bool v = valid && c < m;
+            const uint32_t cc = v ? c : 0u;
+            verlet_consider(ls, box, rb, cj[cc], v, 0u, make_double4(cx[cc], cy[cc], cz[cc], 0.0));
+        }
+        __syncthreads();
+    }
+    if(valid && l == 0) {s.nn[t] = (rb.count < s.p.cap) ? rb.count : s.p.cap;}
+    block_max2_to(valid ? rb.count : 0u, 0u, &s.ctl->maxcount, nullptr);
+    __threadfence_block();     // the row is read back by the lanes that wrote it
+}
+
+// TSP: the system has 3SPN2 terms (their long arithmetic costs the other systems registers).
+template<bool MIXED, bool TSP>
+__global__ void __launch_bounds__(256)
+k_forces(const double4* __restrict__ pos, Box box, SmallForces a)
+{
+    const uint32_t block = blockIdx.x;
+    if(block >= a.noise_begin)
+    {
+        // the next step's draws, ready when k_advance opens it
+        const uint32_t i = (block - a.noise_begin) * blockDim.x + threadIdx.x;
+        if(i < a.n)
+        {
+            double x, y, z;
+            noise3(a.seed, a.sctl->step + a.k + 1, i, x, y, z);
+            a.noise[i] = make_double4(x, y, z, 0.0);
+        }
+        return;
+    }
+    if(block >= a.local_begin)
+    {
+        const uint32_t lb = block - a.local_begin;
+        int si = 0;
+        while(si + 1 < a.nlocal && lb >= a.local[si + 1].block_begin) {++si;}
+        const LocalSeg& s = a.local[si];
+        const uint32_t t = (lb - s.block_begin) * blockDim.x + threadIdx.x;
+        if(t < s.n_terms) {local_term<false, TSP>(s, t, pos, box, a.lidx, a.lpar, a.ldst, a.tf, nullptr);}
+        return;
+    }
+    int si = 0;
+    while(si + 1 < a.nrow && block >= a.row[si + 1].block_begin) {++si;}
+    const RowSeg& s = a.row[si];
+    const uint32_t gt = (block - s.block_begin) * blockDim.x + threadIdx.x;
+    const uint32_t t = gt / s.p.tpp, l = gt % s.p.tpp;
+    const bool valid = t < s.p.np;
+    if(!s.never && margin_after(s.ctl, a.sctl, a.k) < 0) {self_build(s, box, pos, t, l, valid);}
+    if(!valid) {return;}   // whole groups leave together
+    if(TSP && (s.p.kind == kBasePair || s.p.kind == kCrossStack))
+    {
+        TspSeg ts;
+        ts.kind = s.p.kind; ts.np = s.p.np; ts.cap = s.p.cap; ts.tpp = s.p.tpp;
+        ts.spart = s.p.spart; ts.nl = s.p.nl; ts.nn = s.p.nn; ts.ppar = s.p.ppar;
+        ts.acc = s.acc; ts.n = a.n; ts.eout = nullptr;
+        tsp_row<false>(ts, t, l, pos, box);
+    }
+    else if constexpr(MIXED) {pair_row_mixed_store<false>(s.p, t, l, pos, box);}
+    else {pair_row_store<false>(s.p, t, l, pos, box);}
+}
+
+} // mjg

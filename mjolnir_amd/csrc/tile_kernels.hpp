@@ -605,7 +605,6 @@ k_verlet_tiled(const double4* __restrict__ pos, Box box, ListSeg s, uint32_t cap
             {
                 const uint32_t h = u / tpp, l = u % tpp;
                 const uint32_t t = cs + h, ki = c_off[13] + h;
-                if(l == 0) {s.order[t] = s.svals[t];}
                 RowBuild rb;
                 rb.i = sj[ki];
                 rb.ri = make_double4(sx[ki], sy[ki], sz[ki], 0.0);

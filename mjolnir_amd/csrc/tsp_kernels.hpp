@@ -58,8 +58,7 @@ struct TspSeg
 {
     int kind;
     uint32_t np, cap, tpp;
-    const uint32_t* part;
-    const uint32_t* order;
+    const uint32_t* spart;     // particle of each row
     const uint32_t* nl;
     const uint32_t* nn;
     const double* ppar;
@@ -68,14 +67,12 @@ struct TspSeg
     double* eout;              // per row
 };
 
+// one row by the tpp lanes of a group
 template<bool ENERGY>
-__global__ void __launch_bounds__(256)
-k_tsp_pairs(const double4* __restrict__ pos, Box box, TspSeg s)
+__device__ __forceinline__ void tsp_row(const TspSeg& s, uint32_t t, uint32_t l, const double4* __restrict__ pos,
+                                        const Box& box)
 {
-    const uint32_t gt = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t t = gt / s.tpp, l = gt % s.tpp;
-    if(t >= s.np) {return;}   // whole groups leave together
-    const uint32_t i = s.part[s.order[t]];
+    const uint32_t i = s.spart[t];
     const uint32_t* row = s.nl + (size_t)t * s.cap;
     const uint32_t cnt = s.nn[t];
     double e = 0.0;
@@ -96,6 +93,16 @@ k_tsp_pairs(const double4* __restrict__ pos, Box box, TspSeg s)
         for(uint32_t o = s.tpp / 2; o > 0; o >>= 1) {e += __shfl_xor(e, o, kWave);}
         if(l == 0) {s.eout[t] = e;}
     }
+}
+
+template<bool ENERGY>
+__global__ void __launch_bounds__(256)
+k_tsp_pairs(const double4* __restrict__ pos, Box box, TspSeg s)
+{
+    const uint32_t gt = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t t = gt / s.tpp, l = gt % s.tpp;
+    if(t >= s.np) {return;}   // whole groups leave together
+    tsp_row<ENERGY>(s, t, l, pos, box);
 }
 
 __global__ void k_zero_u64(unsigned long long* __restrict__ p, uint32_t n)

@@ -1,0 +1,96 @@
+"""Joined integrator steps (k_advance) and the one-launch forces of small systems with the lists they
+keep (k_forces), against the oracle: the edges of the size rule, both integrators, partitions, and a
+list that outgrows its rows in the middle of a segment."""
+import dataclasses
+import os
+import sys
+
+import numpy as np
+import pytest
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "oracle"))
+pytestmark = pytest.mark.gpu
+
+
+def _follow(spec, steps, precision=0, tol=1e-8, lists=True):
+    """Positions, velocities, forces and the neighbour sets after `steps` steps against the oracle, which
+    takes the same noise.  1e-8 is the bar of the FP64 trajectories (rounding grows by less than 1e4 over
+    a few hundred steps of these systems)."""
+    import oracle
+    from mjolnir_amd import capi
+    e, o = capi.Engine(spec, precision), oracle.OracleEngine(spec)
+    for n in (steps // 3, steps - steps // 3):          # two calls: segments start from a stored state
+        e.step(n)
+        o.step(n)
+    x, v, f = e.state()
+    xo, vo, fo = o.state()
+    d = x - xo
+    if spec.boundary == "periodic":
+        w = spec.upper - spec.lower
+        d -= w * np.round(d / w)
+    scale = np.abs(fo).max()
+    print(f"[gpu] {spec.name}: dx {np.abs(d).max():.1e} dv {np.abs(v - vo).max():.1e} "
+          f"df {np.abs(f - fo).max() / scale:.1e} rebuilds {e.counters()[1]}", flush=True)
+    assert np.abs(d).max() < tol and np.abs(v - vo).max() < tol and np.abs(f - fo).max() < tol * max(1.0, scale)
+    assert e.counters()[0] == steps
+    for g in range(len(spec.global_) if lists else 0):
+        same = np.array_equal(e.pairs(len(spec.local) + g), o.pairs(g))   # the oracle counts globals alone
+        assert same, spec.global_[g].potential
+    return e
+
+
+def _gjf(spec):
+    it = dataclasses.replace(spec.integrator, type="GJFNVTLangevin", coefs=spec.integrator.coefs * spec.mass)
+    return dataclasses.replace(spec, integrator=it)
+
+
+@pytest.mark.parametrize("n,steps", [(65, 150), (257, 150), (1000, 150), (4096, 70), (4097, 70)])
+def test_fluids_at_the_edges_of_the_size_rule(n, steps):
+    from mjolnir_amd import workloads
+    spec = workloads.lj_fluid(n=n, seed=n, margin=0.15 if n < 300 else 0.5)
+    e = _follow(spec, steps)
+    assert e.counters()[1] >= 1
+
+
+@pytest.mark.parametrize("partition", ["CellList", "VerletList", "Naive"])
+def test_partitions(partition):
+    from mjolnir_amd import workloads
+    spec = _gjf(workloads.cg_chain(130, seed=8, max_bend_deg=150.0, margin=0.1))
+    spec.global_ = [dataclasses.replace(g, partition=partition) for g in spec.global_]
+    _follow(spec, 120, tol=1e-7)
+
+
+def test_list_outgrows_its_rows_inside_a_segment():
+    """Two clusters of 48 that drift together: a row holds 47 partners at the start (capacity 64) and 95
+    once the clusters see each other.  The segment then runs again from a list rebuilt at its start, so
+    the later rebuilds fall on other steps than the oracle's and only the trajectory is compared."""
+    from mjolnir_amd import workloads
+    from mjolnir_amd.spec import GlobalSpec, IntegratorSpec, SystemSpec
+    g = np.stack(np.meshgrid(np.arange(4), np.arange(4), np.arange(3), indexing="ij"), -1).reshape(-1, 3) * 1.3
+    pos = np.concatenate([g, g + [16.0, 0.6, 0.6]])
+    vel = np.zeros_like(pos)
+    vel[:48, 0], vel[48:, 0] = 3.5, -3.5
+    n = len(pos)
+    lj = GlobalSpec(potential="LennardJones", participants=np.arange(n), params=np.tile([1.0, 0.02], (n, 1)), cutoff=2.5,
+                    partition="CellList", margin=1.5)
+    spec = SystemSpec(boundary="unlimited", mass=np.ones(n), pos=pos, vel=vel, attributes={"temperature": 1.0},
+                      global_=[lj], integrator=IntegratorSpec("BAOABLangevin", 0.01, np.full(n, 0.01), seed=3),
+                      name="two_clusters")
+    e = _follow(spec, 165, lists=False)
+    per = np.bincount(e.pairs(0).ravel(), minlength=n)
+    assert per.max() > 64
+
+
+@pytest.mark.parametrize("system", ["chain", "dna"])
+def test_mixed_small_systems_follow_fp64(system):
+    """The mixed precision through the same kernels: forces along the way within the mixed bar of the FP64
+    engine's (1e-5 of the RMS force) after 60 steps of one noise stream."""
+    from mjolnir_amd import capi, workloads
+    spec = workloads.cg_chain(700, seed=9, max_bend_deg=150.0) if system == "chain" else workloads.dna_duplex(40, seed=5)
+    a, b = capi.Engine(spec, capi.FP64), capi.Engine(spec, capi.FP32_FIXED)
+    a.step(60)
+    b.step(60)
+    fa, fb = a.state()[2], b.state()[2]
+    rms = np.sqrt(np.mean(fa ** 2))
+    print(f"[gpu] {system} mixed vs FP64: {np.sqrt(np.mean((fa - fb) ** 2)) / rms:.1e}", flush=True)
+    assert np.sqrt(np.mean((fa - fb) ** 2)) < 1e-5 * rms
