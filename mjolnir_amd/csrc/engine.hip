@@ -1439,23 +1439,18 @@ void Engine::launch_advance(uint32_t k, bool last)
     a.box = box_;
     a.n = (uint32_t)n_;
     a.k = k;
-    const dim3 grid(blocks_for(n_, 256)), block(256);
-    const bool gjf = (integ_ == MJG_INTEG_GJF);
-    if(k == 0)
-    {
-        if(gjf) {hipLaunchKernelGGL((k_advance<true, true, false>), grid, block, 0, stream_, a);}
-        else {hipLaunchKernelGGL((k_advance<false, true, false>), grid, block, 0, stream_, a);}
-    }
-    else if(last)
-    {
-        if(gjf) {hipLaunchKernelGGL((k_advance<true, false, true>), grid, block, 0, stream_, a);}
-        else {hipLaunchKernelGGL((k_advance<false, false, true>), grid, block, 0, stream_, a);}
-    }
-    else
-    {
-        if(gjf) {hipLaunchKernelGGL((k_advance<true, false, false>), grid, block, 0, stream_, a);}
-        else {hipLaunchKernelGGL((k_advance<false, false, false>), grid, block, 0, stream_, a);}
-    }
+    const bool gjf = (integ_ == MJG_INTEG_GJF), first = (k == 0);
+    auto go = [&](auto staged) {
+        constexpr bool S = decltype(staged)::value;
+        const dim3 grid(blocks_for(n_, S ? kStagedParticles : 256)), block(256);
+        if(gjf && first) {hipLaunchKernelGGL((k_advance<true, true, false, S>), grid, block, 0, stream_, a);}
+        else if(gjf && last) {hipLaunchKernelGGL((k_advance<true, false, true, S>), grid, block, 0, stream_, a);}
+        else if(gjf) {hipLaunchKernelGGL((k_advance<true, false, false, S>), grid, block, 0, stream_, a);}
+        else if(first) {hipLaunchKernelGGL((k_advance<false, true, false, S>), grid, block, 0, stream_, a);}
+        else if(last) {hipLaunchKernelGGL((k_advance<false, false, true, S>), grid, block, 0, stream_, a);}
+        else {hipLaunchKernelGGL((k_advance<false, false, false, S>), grid, block, 0, stream_, a);}
+    };
+    if(local_blocks_ > 0 && small_) {go(std::true_type{});} else {go(std::false_type{});}
 }
 
 // The forces of step k: one launch for a small system, else the rebuild pipeline and the
@@ -1488,7 +1483,7 @@ void Engine::launch_step_forces(uint32_t k)
             r.nl = g.d_nl; r.nn = g.d_nn;
             r.part = g.d_part; r.pslot = g.d_pslot; r.mol = g.d_mol; r.ex_start = g.d_ex_start; r.ex = g.d_ex;
             r.rule = g.rule;
-            block += blocks_for((size_t)r.p.np * r.p.tpp, 256);
+            block += blocks_for((size_t)r.p.np * r.p.tpp * (g.pot == kCrossStack ? 4 : 1), 256);
         }
     }
     a.local_begin = block;

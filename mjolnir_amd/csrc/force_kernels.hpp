@@ -431,13 +431,38 @@ struct PairSegTable
 // little else.
 constexpr int kPairBatch = 4;
 
-template<int KIND, bool ENERGY>
-__device__ __forceinline__ void pair_row(const PairSeg& s, uint32_t t, uint32_t l, const double4* __restrict__ pos,
-                                         const Box& box, double& fx, double& fy, double& fz, double& e, uint32_t& i)
+// What a lane needs of its row before any position: the particle, the row's length and the lane's
+// first words, read together (a word past the row's end is dropped by length afterwards).
+struct RowHead
 {
-    i = s.spart[t];
-    const uint32_t cnt = s.nn[t];
+    uint32_t i, cnt;
+    uint32_t w[kPairBatch];
+};
+__device__ __forceinline__ RowHead row_head(const PairSeg& s, uint32_t t, uint32_t l)
+{
+    RowHead h;
+    h.i = s.spart[t];
+    h.cnt = s.nn[t];
     const uint32_t* row = s.nl + (size_t)t * s.cap;
+#pragma unroll
+    for(int m = 0; m < kPairBatch; ++m)
+    {
+        const uint32_t k = l + m * s.tpp;
+        h.w[m] = row[(k < s.cap) ? k : 0u];
+    }
+    return h;
+}
+
+template<int KIND, bool ENERGY>
+__device__ __forceinline__ void pair_row(const PairSeg& s, const RowHead& h, uint32_t t, uint32_t l,
+                                         const double4* __restrict__ pos, const Box& box, double& fx, double& fy,
+                                         double& fz, double& e)
+{
+    const uint32_t i = h.i, cnt = h.cnt;
+    const uint32_t* row = s.nl + (size_t)t * s.cap;
+    uint32_t w[kPairBatch];
+#pragma unroll
+    for(int m = 0; m < kPairBatch; ++m) {w[m] = h.w[m];}
     const double4 ri = pos[i];
     RegPar par;
     load_par<KIND>(s.ppar, i, par.a0, par.a1);
@@ -450,7 +475,14 @@ __device__ __forceinline__ void pair_row(const PairSeg& s, uint32_t t, uint32_t 
         for(int m = 0; m < kPairBatch; ++m)
         {
             const uint32_t k = k0 + m * s.tpp;
-            j[m] = (k < cnt) ? row[k] : i;
+            j[m] = (k < cnt) ? w[m] : i;
+        }
+        // the next batch's words are on their way while this one is computed
+#pragma unroll
+        for(int m = 0; m < kPairBatch; ++m)
+        {
+            const uint32_t k = k0 + (kPairBatch + m) * s.tpp;
+            w[m] = (k < cnt) ? row[k] : 0u;
         }
 #pragma unroll
         for(int m = 0; m < kPairBatch; ++m) {rj[m] = pos[j[m]]; load_par<KIND>(s.ppar, j[m], p0[m], p1[m]);}
@@ -468,15 +500,15 @@ __device__ __forceinline__ void pair_row(const PairSeg& s, uint32_t t, uint32_t 
 
 // one row by the tpp lanes of a group: its force (and energy) stored by lane 0
 template<bool ENERGY>
-__device__ __forceinline__ void pair_row_store(const PairSeg& s, uint32_t t, uint32_t l, const double4* __restrict__ pos,
-                                               const Box& box)
+__device__ __forceinline__ void pair_row_store(const PairSeg& s, const RowHead& h, uint32_t t, uint32_t l,
+                                               const double4* __restrict__ pos, const Box& box)
 {
     double fx = 0, fy = 0, fz = 0, e = 0;
-    uint32_t i = 0;
-    if(s.kind == kPairLJ) {pair_row<kPairLJ, ENERGY>(s, t, l, pos, box, fx, fy, fz, e, i);}
-    else if(s.kind == kPairEV) {pair_row<kPairEV, ENERGY>(s, t, l, pos, box, fx, fy, fz, e, i);}
-    else if(s.kind == kPair3SPN2EV) {pair_row<kPair3SPN2EV, ENERGY>(s, t, l, pos, box, fx, fy, fz, e, i);}
-    else {pair_row<kPairDH, ENERGY>(s, t, l, pos, box, fx, fy, fz, e, i);}
+    const uint32_t i = h.i;
+    if(s.kind == kPairLJ) {pair_row<kPairLJ, ENERGY>(s, h, t, l, pos, box, fx, fy, fz, e);}
+    else if(s.kind == kPairEV) {pair_row<kPairEV, ENERGY>(s, h, t, l, pos, box, fx, fy, fz, e);}
+    else if(s.kind == kPair3SPN2EV) {pair_row<kPair3SPN2EV, ENERGY>(s, h, t, l, pos, box, fx, fy, fz, e);}
+    else {pair_row<kPairDH, ENERGY>(s, h, t, l, pos, box, fx, fy, fz, e);}
     for(uint32_t o = s.tpp / 2; o > 0; o >>= 1)
     {
         fx += __shfl_xor(fx, o, kWave);
@@ -501,7 +533,7 @@ k_pairs(const double4* __restrict__ pos, Box box, PairSegTable tab)
     const uint32_t gt = (blockIdx.x - s.block_begin) * blockDim.x + threadIdx.x;
     const uint32_t t = gt / s.tpp, l = gt % s.tpp;
     if(t >= s.np) {return;}   // whole groups leave together
-    pair_row_store<ENERGY>(s, t, l, pos, box);
+    pair_row_store<ENERGY>(s, row_head(s, t, l), t, l, pos, box);
 }
 
 // ------------------------------------------------------------------------------------
@@ -592,14 +624,16 @@ __device__ __forceinline__ bool pair_term_f32(const PairConstsF& K, const PairPa
 }
 
 template<int KIND, bool ENERGY>
-__device__ __forceinline__ void pair_row_mixed(const PairSeg& s, uint32_t t, uint32_t l, const double4* __restrict__ pos,
-                                               const Box& box, long long& ax, long long& ay, long long& az, double& e,
-                                               uint32_t& i)
+__device__ __forceinline__ void pair_row_mixed(const PairSeg& s, const RowHead& h, uint32_t t, uint32_t l,
+                                               const double4* __restrict__ pos, const Box& box, long long& ax,
+                                               long long& ay, long long& az, double& e)
 {
     const PairConstsF K = pair_consts_f(s.pp);
-    i = s.spart[t];
-    const uint32_t cnt = s.nn[t];
+    const uint32_t i = h.i, cnt = h.cnt;
     const uint32_t* row = s.nl + (size_t)t * s.cap;
+    uint32_t w[kPairBatch];
+#pragma unroll
+    for(int m = 0; m < kPairBatch; ++m) {w[m] = h.w[m];}
     const double4 ri = pos[i];
     RegPar par;
     load_par<KIND>(s.ppar, i, par.a0, par.a1);
@@ -612,7 +646,14 @@ __device__ __forceinline__ void pair_row_mixed(const PairSeg& s, uint32_t t, uin
         for(int m = 0; m < kPairBatch; ++m)
         {
             const uint32_t k = k0 + m * s.tpp;
-            j[m] = (k < cnt) ? row[k] : i;
+            j[m] = (k < cnt) ? w[m] : i;
+        }
+        // the next batch's words are on their way while this one is computed
+#pragma unroll
+        for(int m = 0; m < kPairBatch; ++m)
+        {
+            const uint32_t k = k0 + (kPairBatch + m) * s.tpp;
+            w[m] = (k < cnt) ? row[k] : 0u;
         }
 #pragma unroll
         for(int m = 0; m < kPairBatch; ++m) {rj[m] = pos[j[m]]; load_par<KIND>(s.ppar, j[m], p0[m], p1[m]);}
@@ -640,16 +681,16 @@ __device__ __forceinline__ long long shfl_xor_ll(long long v, int o)
 }
 
 template<bool ENERGY>
-__device__ __forceinline__ void pair_row_mixed_store(const PairSeg& s, uint32_t t, uint32_t l,
+__device__ __forceinline__ void pair_row_mixed_store(const PairSeg& s, const RowHead& h, uint32_t t, uint32_t l,
                                                      const double4* __restrict__ pos, const Box& box)
 {
     long long ax = 0, ay = 0, az = 0;
     double e = 0;
-    uint32_t i = 0;
-    if(s.kind == kPairLJ) {pair_row_mixed<kPairLJ, ENERGY>(s, t, l, pos, box, ax, ay, az, e, i);}
-    else if(s.kind == kPairEV) {pair_row_mixed<kPairEV, ENERGY>(s, t, l, pos, box, ax, ay, az, e, i);}
-    else if(s.kind == kPair3SPN2EV) {pair_row_mixed<kPair3SPN2EV, ENERGY>(s, t, l, pos, box, ax, ay, az, e, i);}
-    else {pair_row_mixed<kPairDH, ENERGY>(s, t, l, pos, box, ax, ay, az, e, i);}
+    const uint32_t i = h.i;
+    if(s.kind == kPairLJ) {pair_row_mixed<kPairLJ, ENERGY>(s, h, t, l, pos, box, ax, ay, az, e);}
+    else if(s.kind == kPairEV) {pair_row_mixed<kPairEV, ENERGY>(s, h, t, l, pos, box, ax, ay, az, e);}
+    else if(s.kind == kPair3SPN2EV) {pair_row_mixed<kPair3SPN2EV, ENERGY>(s, h, t, l, pos, box, ax, ay, az, e);}
+    else {pair_row_mixed<kPairDH, ENERGY>(s, h, t, l, pos, box, ax, ay, az, e);}
     for(uint32_t o = s.tpp / 2; o > 0; o >>= 1)
     {
         ax += shfl_xor_ll(ax, (int)o);
@@ -678,7 +719,7 @@ k_pairs_mixed(const double4* __restrict__ pos, Box box, PairSegTable tab)
     const uint32_t gt = (blockIdx.x - s.block_begin) * blockDim.x + threadIdx.x;
     const uint32_t t = gt / s.tpp, l = gt % s.tpp;
     if(t >= s.np) {return;}   // whole groups leave together
-    pair_row_mixed_store<ENERGY>(s, t, l, pos, box);
+    pair_row_mixed_store<ENERGY>(s, row_head(s, t, l), t, l, pos, box);
 }
 
 // The force on one particle: its local-term slots (in interaction, term order) plus every pair
@@ -692,15 +733,24 @@ struct GatherArgs
     unsigned long long* acc[kMaxPairSegs];
     int ng;
 };
+// staged: the block's slots in LDS, from slot `first` on (null: none)
 template<bool CLEAR>
-__device__ __forceinline__ void gather_force(const GatherArgs& a, uint32_t n, uint32_t i, double& x, double& y, double& z)
+__device__ __forceinline__ void gather_force(const GatherArgs& a, uint32_t n, uint32_t i, double& x, double& y, double& z,
+                                             const double* staged = nullptr, uint32_t first = 0)
 {
     x = 0; y = 0; z = 0;
     if(a.gstart != nullptr)
     {
-        // four slots' loads in flight at a time, added in order
         const uint32_t b = a.gstart[i], e = a.gstart[i + 1];
-        for(uint32_t k = b; k < e; k += 4)
+        if(staged != nullptr)
+        {
+            for(uint32_t k = 3 * (b - first); k < 3 * (e - first); k += 3)
+            {
+                x += staged[k]; y += staged[k + 1]; z += staged[k + 2];
+            }
+        }
+        // four slots' loads in flight at a time, added in order
+        else for(uint32_t k = b; k < e; k += 4)
         {
             double v[12];
 #pragma unroll

@@ -37,7 +37,9 @@ struct SelfLists
 // margin left after the step's largest displacement, below zero when the list must be rebuilt.
 __device__ __forceinline__ double margin_after(const ListCtl* ctl, const StepCtl* sctl, uint32_t k)
 {
-    return ctl->margin - 2 * sqrt(__longlong_as_double((long long)sctl->maxdisp2[(sctl->step + k) & 1]));
+    // both slots are read with the step count, not after it
+    const unsigned long long d0 = sctl->maxdisp2[0], d1 = sctl->maxdisp2[1];
+    return ctl->margin - 2 * sqrt(__longlong_as_double((long long)(((sctl->step + k) & 1) ? d1 : d0)));
 }
 
 struct AdvanceArgs
@@ -64,14 +66,44 @@ struct AdvanceArgs
     int nlists;
 };
 
+// STAGED: the system has local terms.  A block of 256 threads then serves 64 particles and brings their
+// term-force slots, one contiguous run, to LDS in a single round of loads (a thread that walked its
+// own dozen slots waited for three or four rounds: k_advance of a 1000-bead chain 6.5 us, of a
+// fluid of that size 3.9).
 // FIRST: opens step 0 from the stored force.  LAST: closes step k - 1 only, stores the force,
 // advances the step count by k and reports to the host.
-template<bool GJF, bool FIRST, bool LAST>
+constexpr uint32_t kStagedParticles = 64;
+constexpr uint32_t kStagedRounds = 12;       // words a thread brings; longer runs are read where they lie
+template<bool GJF, bool FIRST, bool LAST, bool STAGED>
 __global__ void __launch_bounds__(256)
 k_advance(AdvanceArgs a)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t per = STAGED ? kStagedParticles : blockDim.x;
+    const uint32_t i = (threadIdx.x < per) ? blockIdx.x * per + threadIdx.x : a.n;
     const uint64_t step0 = a.ctl->step;
+    const double* slots = nullptr;
+    uint32_t slot0 = 0;
+    if constexpr(STAGED && !FIRST)
+    {
+        __shared__ double staged[kStagedRounds * 256];
+        const uint32_t i0 = blockIdx.x * per, i1 = (i0 + per < a.n) ? i0 + per : a.n;
+        const uint32_t b = a.g.gstart[i0], words = 3 * (a.g.gstart[i1] - b);
+        if(words <= kStagedRounds * 256)
+        {
+            double v[kStagedRounds];
+#pragma unroll
+            for(uint32_t m = 0; m < kStagedRounds; ++m)
+            {
+                const uint32_t q = m * 256 + threadIdx.x;
+                v[m] = (q < words) ? a.g.tf[3 * (size_t)b + q] : 0.0;
+            }
+#pragma unroll
+            for(uint32_t m = 0; m < kStagedRounds; ++m) {staged[m * 256 + threadIdx.x] = v[m];}
+            slots = staged;
+            slot0 = b;
+        }
+        __syncthreads();
+    }
     if constexpr(!FIRST)
     {
         // the previous step's skin decision, taken by every block of its k_forces, is made final
@@ -109,7 +141,7 @@ k_advance(AdvanceArgs a)
         if constexpr(FIRST) {const double4 f = a.force[i]; fx = f.x; fy = f.y; fz = f.z;}
         else
         {
-            gather_force<true>(a.g, a.n, i, fx, fy, fz);
+            gather_force<true>(a.g, a.n, i, fx, fy, fz, slots, slot0);
             // closing half-kick (BAOABLangevinIntegrator.hpp:222-229, GJFNVTLangevinIntegrator.hpp:222-229)
             const double hrm = a.halfdt * rm;
             v.x += hrm * fx; v.y += hrm * fy; v.z += hrm * fz;
@@ -233,51 +265,124 @@ struct SmallForces
     uint32_t n, k;
 };
 constexpr uint32_t kScanTile = 256;   // candidates staged at a time by a rebuild
+constexpr uint32_t kScanEx = 4096;    // exclusions staged by a block, shared out over its rows
 
-// The rows of one block found among all participants, in participant order (the pairs and the test
-// are k_verlet's).  Every thread of the block calls it; `valid`: the thread's row exists.
+// The rows of one block found among all participants, in participant order; the pairs are k_verlet's
+// (the same distance test, pair_allowed's rules).  A candidate near enough used to read the participant,
+// base and exclusion tables in a dependent chain of about 3 us, on nearly every round of a chain's or
+// a duplex's rows (251 us a rebuild of the 200-bp duplex); here a tile's tables are staged with its
+// positions, loaded while the tile before is tested, and a row keeps its own exclusions in LDS (an
+// exclusion holds both ways, so the owner's list decides).  Every thread of the block calls it;
+// `valid`: the thread's row exists.
 __device__ __forceinline__ void self_build(const RowSeg& s, const Box& box, const double4* __restrict__ pos, uint32_t t,
                                            uint32_t l, bool valid)
 {
     __shared__ double cx[kScanTile], cy[kScanTile], cz[kScanTile];
-    __shared__ uint32_t cj[kScanTile];
+    __shared__ uint32_t cj[kScanTile], cslot[kScanTile], cmol[kScanTile];
+    __shared__ int cbase[kScanTile];
+    __shared__ uint32_t ex[kScanEx];
     const uint32_t tid = threadIdx.x, lane = tid % kWave;
-    const uint32_t np = s.p.np, tpp = s.p.tpp;
-    ListSeg ls{};
-    ls.cap = s.p.cap;
-    ls.pslot = s.pslot; ls.mol = s.mol; ls.ex_start = s.ex_start; ls.ex = s.ex;
-    ls.rule = s.rule;
-    RowBuild rb;
-    rb.i = valid ? s.p.spart[t] : 0u;
-    rb.ri = pos[rb.i];
-    rb.gmask = group_mask_of(tpp, lane);
-    rb.below = rb.gmask & ((1ull << lane) - 1ull);
-    rb.count = 0;
-    rb.row = s.nl + (size_t)(valid ? t : 0u) * s.p.cap;
-    rb.row16 = nullptr;
+    const uint32_t np = s.p.np, tpp = s.p.tpp, cap = s.p.cap;
+    const ListRule& rule = s.rule;
+    const uint32_t i = valid ? s.p.spart[t] : 0u;
+    const double4 ri = pos[i];
+    const uint32_t islot = s.pslot[i], imol = rule.ignore_mol ? s.mol[i] : 0u;
+    const int ibase = rule.base_rule ? (int)rule.base_par[(size_t)i * rule.base_stride] : 0;
+    const uint64_t gmask = group_mask_of(tpp, lane), below = gmask & ((1ull << lane) - 1ull);
+    // the row's exclusions: those within 32 indices of i as bits, the first `excap` of the others in
+    // LDS, any more read where they lie
+    const uint32_t exb = s.ex_start[i], exn = rule.simple ? 0u : s.ex_start[i + 1] - exb;
+    const uint32_t excap = kScanEx / (blockDim.x / tpp), exo = (tid / tpp) * excap;
+    unsigned long long near = 0;
+    uint32_t nfar = 0, over = exn;
+    for(uint32_t k0 = 0; k0 < exn; k0 += tpp)
+    {
+        const uint32_t k = k0 + l;
+        const uint32_t e = (k < exn) ? s.ex[exb + k] : i;
+        const uint32_t d = e - i + 32u;
+        const bool far = d >= 64u;
+        if(!far) {near |= 1ull << d;}
+        const uint64_t f = __ballot(far) & gmask;
+        const uint32_t at = nfar + (uint32_t)__popcll(f & below);
+        if(far && at < excap) {ex[exo + at] = e;}
+        nfar += (uint32_t)__popcll(f);
+        if(nfar > excap && over == exn) {over = k0;}       // words from here on may not be staged
+    }
+    for(uint32_t o = tpp / 2; o > 0; o >>= 1) {near |= (unsigned long long)__shfl_xor((long long)near, o, kWave);}
+    const uint32_t exl = (nfar < excap) ? nfar : excap;
+    uint32_t* row = s.nl + (size_t)(valid ? t : 0u) * cap;
+    uint32_t count = 0;
+
+    double4 nr = ri;
+    uint32_t nj = 0, nslot = 0, nmol = 0;
+    int nbase = 0;
+    auto fetch = [&](uint32_t base) {
+        const uint32_t q = base + tid;
+        if(q >= np) {return;}
+        nj = s.part[q];
+        nr = pos[nj];
+        nslot = s.pslot[nj];
+        if(rule.ignore_mol) {nmol = s.mol[nj];}
+        if(rule.base_rule) {nbase = (int)rule.base_par[(size_t)nj * rule.base_stride];}
+    };
+    fetch(0);
     for(uint32_t base = 0; base < np; base += kScanTile)
     {
-        const uint32_t q = base + tid;
-        if(q < np)
-        {
-            const uint32_t j = s.part[q];
-            const double4 r = pos[j];
-            cx[tid] = r.x; cy[tid] = r.y; cz[tid] = r.z; cj[tid] = j;
-        }
         __syncthreads();
+        cx[tid] = nr.x; cy[tid] = nr.y; cz[tid] = nr.z;
+        cj[tid] = nj; cslot[tid] = nslot; cmol[tid] = nmol; cbase[tid] = nbase;
+        __syncthreads();
+        fetch(base + kScanTile);
         const uint32_t m = (np - base < kScanTile) ? np - base : kScanTile;
         for(uint32_t b = 0; b < m; b += tpp)
         {
             const uint32_t c = b + l;
-            const bool v = valid && c < m;
-            const uint32_t cc = v ? c : 0u;
-            verlet_consider(ls, box, rb, cj[cc], v, 0u, make_double4(cx[cc], cy[cc], cz[cc], 0.0));
+            bool accept = valid && c < m;
+            const uint32_t q = accept ? c : 0u;
+            const uint32_t j = cj[q];
+            accept = accept && j != i;
+            const bool up = i < j;
+            if(accept && rule.use_distance)
+            {
+                // the reference measures the pair from its lower index (same operands, same order)
+                const double4 rj = make_double4(cx[q], cy[q], cz[q], 0.0);
+                const double4 from = up ? ri : rj, to = up ? rj : ri;
+                double dx, dy, dz;
+                adjust_direction(box, from.x, from.y, from.z, to.x, to.y, to.z, dx, dy, dz);
+                accept = length_sq(dx, dy, dz) < rule.r_list2;
+            }
+            if(accept)
+            {
+                const uint32_t slo = up ? islot : cslot[q], shi = up ? cslot[q] : islot;
+                accept = rule.pairwise ? slo <= shi : slo != rule.last_slot;
+                if(rule.ignore_mol == 1) {accept = accept && imol != cmol[q];}
+                if(rule.ignore_mol == 2) {accept = accept && imol == cmol[q];}
+                const int jbase = cbase[q];
+                if(rule.base_rule == 1)
+                {
+                    accept = accept && !(ibase >= 2 && jbase >= 2 && complementary_bases(ibase - 2, jbase - 2));
+                }
+                else if(rule.base_rule == 2) {accept = accept && complementary_bases(ibase, jbase);}
+                const uint32_t d = j - i + 32u;
+                if(d < 64u) {accept = accept && ((near >> d) & 1ull) == 0ull;}
+                else
+                {
+                    for(uint32_t k = 0; accept && k < exl; ++k) {accept = ex[exo + k] != j;}
+                    for(uint32_t k = over; accept && k < exn; ++k) {accept = s.ex[exb + k] != j;}
+                }
+            }
+            const uint64_t took = __ballot(accept) & gmask;
+            if(accept)
+            {
+                const uint32_t k = count + (uint32_t)__popcll(took & below);
+                if(k < cap) {row[k] = j;}
+            }
+            count += (uint32_t)__popcll(took);
         }
-        __syncthreads();
     }
-    if(valid && l == 0) {s.nn[t] = (rb.count < s.p.cap) ? rb.count : s.p.cap;}
-    block_max2_to(valid ? rb.count : 0u, 0u, &s.ctl->maxcount, nullptr);
-    __threadfence_block();     // the row is read back by the lanes that wrote it
+    if(valid && l == 0) {s.nn[t] = (count < cap) ? count : cap;}
+    block_max2_to(valid ? count : 0u, 0u, &s.ctl->maxcount, nullptr);
+    __threadfence_block();     // the rows are read back by the block that wrote them
 }
 
 // TSP: the system has 3SPN2 terms (their long arithmetic costs the other systems registers).
@@ -311,10 +416,20 @@ k_forces(const double4* __restrict__ pos, Box box, SmallForces a)
     int si = 0;
     while(si + 1 < a.nrow && block >= a.row[si + 1].block_begin) {++si;}
     const RowSeg& s = a.row[si];
-    const uint32_t gt = (block - s.block_begin) * blockDim.x + threadIdx.x;
-    const uint32_t t = gt / s.p.tpp, l = gt % s.p.tpp;
+    // a row's lanes: tpp, four times as many for cross stacking (one pair on four lanes); a rebuild
+    // takes tpp of them, the lanes of one wave
+    const uint32_t lanes = (TSP && s.p.kind == kCrossStack) ? 4 * s.p.tpp : s.p.tpp;
+    const uint32_t rows = 256 / lanes, row0 = (block - s.block_begin) * rows;
+    const uint32_t t = row0 + threadIdx.x / lanes, l = threadIdx.x % lanes;
     const bool valid = t < s.p.np;
-    if(!s.never && margin_after(s.ctl, a.sctl, a.k) < 0) {self_build(s, box, pos, t, l, valid);}
+    // the row's head is on its way while the skin decision's words are
+    RowHead h = row_head(s.p, valid ? t : 0u, l);
+    if(!s.never && margin_after(s.ctl, a.sctl, a.k) < 0)
+    {
+        const uint32_t r = threadIdx.x / s.p.tpp;
+        self_build(s, box, pos, row0 + r, threadIdx.x % s.p.tpp, r < rows && row0 + r < s.p.np);
+        h = row_head(s.p, valid ? t : 0u, l);
+    }
     if(!valid) {return;}   // whole groups leave together
     if(TSP && (s.p.kind == kBasePair || s.p.kind == kCrossStack))
     {
@@ -322,10 +437,11 @@ k_forces(const double4* __restrict__ pos, Box box, SmallForces a)
         ts.kind = s.p.kind; ts.np = s.p.np; ts.cap = s.p.cap; ts.tpp = s.p.tpp;
         ts.spart = s.p.spart; ts.nl = s.p.nl; ts.nn = s.p.nn; ts.ppar = s.p.ppar;
         ts.acc = s.acc; ts.n = a.n; ts.eout = nullptr;
-        tsp_row<false>(ts, t, l, pos, box);
+        if(s.p.kind == kBasePair) {tsp_row<false, 1>(ts, t, l, pos, box);}
+        else {tsp_row<false, 4>(ts, t, l, pos, box);}
     }
-    else if constexpr(MIXED) {pair_row_mixed_store<false>(s.p, t, l, pos, box);}
-    else {pair_row_store<false>(s.p, t, l, pos, box);}
+    else if constexpr(MIXED) {pair_row_mixed_store<false>(s.p, h, t, l, pos, box);}
+    else {pair_row_store<false>(s.p, h, t, l, pos, box);}
 }
 
 } // mjg

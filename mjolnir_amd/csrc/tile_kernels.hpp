@@ -152,12 +152,13 @@ __device__ __forceinline__ void tile_rows_global(const TileSeg& s, const double4
     for(uint32_t u = threadIdx.x; u < nhome * tpp; u += kTileThreads)
     {
         const uint32_t t = cs + u / tpp, l = u % tpp;
-        uint32_t i = 0;
+        const RowHead hd = row_head(ps, t, l);
+        const uint32_t i = hd.i;
         double e = 0;
         if constexpr(MIXED)
         {
             long long ax = 0, ay = 0, az = 0;
-            pair_row_mixed<KIND, ENERGY>(ps, t, l, pos, box, ax, ay, az, e, i);
+            pair_row_mixed<KIND, ENERGY>(ps, hd, t, l, pos, box, ax, ay, az, e);
             for(uint32_t o = tpp / 2; o > 0; o >>= 1)
             {
                 ax += shfl_xor_ll(ax, (int)o);
@@ -179,7 +180,7 @@ __device__ __forceinline__ void tile_rows_global(const TileSeg& s, const double4
         else
         {
             double fx = 0, fy = 0, fz = 0;
-            pair_row<KIND, ENERGY>(ps, t, l, pos, box, fx, fy, fz, e, i);
+            pair_row<KIND, ENERGY>(ps, hd, t, l, pos, box, fx, fy, fz, e);
             for(uint32_t o = tpp / 2; o > 0; o >>= 1)
             {
                 fx += __shfl_xor(fx, o, kWave);

@@ -67,13 +67,16 @@ struct TspSeg
     double* eout;              // per row
 };
 
-// one row by the tpp lanes of a group
-template<bool ENERGY>
+// One row by `tpp` times QUAD lanes.  QUAD = 4 (cross stacking without energies): four lanes share a
+// pair, each with one of its elements.
+template<bool ENERGY, int QUAD>
 __device__ __forceinline__ void tsp_row(const TspSeg& s, uint32_t t, uint32_t l, const double4* __restrict__ pos,
                                         const Box& box)
 {
-    const uint32_t i = s.spart[t];
     const uint32_t* row = s.nl + (size_t)t * s.cap;
+    const uint32_t k0 = l / QUAD;
+    const uint32_t first = row[(k0 < s.cap) ? k0 : 0u];      // with the row's particle and length
+    const uint32_t i = s.spart[t];
     const uint32_t cnt = s.nn[t];
     double e = 0.0;
     tsp::GlobalFixAcc acc;
@@ -81,11 +84,12 @@ __device__ __forceinline__ void tsp_row(const TspSeg& s, uint32_t t, uint32_t l,
     acc.box = box;
     acc.acc = s.acc;
     acc.flag = s.acc + 3 * (size_t)s.n;
-    for(uint32_t k = l; k < cnt; k += s.tpp)
+    for(uint32_t k = k0; k < cnt; k += s.tpp)
     {
-        const uint32_t j = row[k];
+        const uint32_t j = (k == k0) ? first : row[k];
         if(j <= i) {continue;}
-        if(s.kind == kBasePair) {tsp::base_pair<double, ENERGY>(i, j, acc, s.ppar, e);}
+        if constexpr(QUAD == 4) {tsp::cross_stack_element(i, j, (int)(l % 4), acc, s.ppar);}
+        else if(s.kind == kBasePair) {tsp::base_pair<double, ENERGY>(i, j, acc, s.ppar, e);}
         else {tsp::cross_stack<double, ENERGY>(i, j, acc, s.ppar, e);}
     }
     if(ENERGY)
@@ -102,7 +106,7 @@ k_tsp_pairs(const double4* __restrict__ pos, Box box, TspSeg s)
     const uint32_t gt = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t t = gt / s.tpp, l = gt % s.tpp;
     if(t >= s.np) {return;}   // whole groups leave together
-    tsp_row<ENERGY>(s, t, l, pos, box);
+    tsp_row<ENERGY, 1>(s, t, l, pos, box);
 }
 
 __global__ void k_zero_u64(unsigned long long* __restrict__ p, uint32_t n)

@@ -434,5 +434,51 @@ __device__ void cross_stack(uint32_t Bi, uint32_t Bj, const Acc& acc, const doub
     if(Bj5e) {acc.add((uint32_t)pj[2], f_Bj5);}
 }
 
+// One of the four elements of a cross-stacking pair (q: the 5' neighbour of Bj, of Bi, the 3' neighbour
+// of Bi, of Bj, the order cross_stack takes them in), for four lanes that share the pair: an element is
+// a chain of FP64 transcendentals of its own behind a short common part, and the four in a row were
+// the longest chain of a duplex's force call.  The element's operands are selected, not branched to,
+// so the four lanes run together.
+template<typename Acc>
+__device__ __forceinline__ void cross_stack_element(uint32_t Bi, uint32_t Bj, int q, const Acc& acc,
+                                                    const double* __restrict__ ppar)
+{
+    using R = double;
+    const R K_BP = 12.0, piK_BP = kPi / 12.0, cutoff_sq = 18.0 * 18.0;
+    const double* pi_ = ppar + 4 * (size_t)Bi;
+    const double* pj = ppar + 4 * (size_t)Bj;
+    const bool own = (q == 0 || q == 3);                 // element at Bi with a neighbour of Bj
+    const double nb = (own ? pj : pi_)[q < 2 ? 2 : 3];
+    const V3<R> Bij = acc.disp(Bi, Bj);
+    if(lsq(Bij) > cutoff_sq || !(nb >= 0)) {return;}
+    const int bi = (int)pi_[0], bj = (int)pj[0];
+    const uint32_t Bn = (uint32_t)nb, Si = (uint32_t)pi_[1], Sj = (uint32_t)pj[1];
+    const int cs = ((own ? bi : bj) << 2 | (int)ppar[4 * (size_t)Bn]) + (q < 2 ? 0 : 16);
+    const V3<R> SBi = acc.disp(Si, Bi), SBj = acc.disp(Sj, Bj);
+    const R rlSBi = 1 / sqrt(lsq(SBi)), rlSBj = 1 / sqrt(lsq(SBj));
+    const V3<R> BSi_reg = (-rlSBi) * SBi, BSj_reg = (-rlSBj) * SBj;
+    const R cos_theta3 = dot(BSi_reg, BSj_reg);
+    const R theta3 = acos(clamp1(cos_theta3));
+    const R th3_0 = cs_theta3(bp_kind(bi));
+    const R f3 = f_mod(K_BP, piK_BP, theta3, th3_0);
+    if(f3 == 0) {return;}
+    const R df3 = df_mod(K_BP, piK_BP, theta3, th3_0);
+    const R sin_theta3 = sin(theta3);
+    const R rsin_theta3 = sin_theta3 > kTol ? 1 / sin_theta3 : 1.0 / kTol;
+    const V3<R> fBi_t3 = (rsin_theta3 * rlSBi) * (BSj_reg - cos_theta3 * BSi_reg);
+    const V3<R> fBj_t3 = (rsin_theta3 * rlSBj) * (BSi_reg - cos_theta3 * BSj_reg);
+    const V3<R> fSi_t3 = (R)(-1) * fBi_t3, fSj_t3 = (R)(-1) * fBj_t3;
+    const V3<R> zero{0, 0, 0};
+    V3<R> f_S1 = zero, f_B1 = zero, f_S2 = zero, f_B2 = zero, f_Bn = zero;
+    cs_element<R, false>(cs, f3, df3, acc, own ? Bi : Bj, Bn, own ? SBi : SBj, own ? rlSBi : rlSBj,
+                         own ? BSi_reg : BSj_reg, own ? fSi_t3 : fSj_t3, own ? fBi_t3 : fBj_t3, own ? fSj_t3 : fSi_t3,
+                         own ? fBj_t3 : fBi_t3, f_S1, f_B1, f_S2, f_B2, f_Bn);
+    acc.add(own ? Si : Sj, f_S1);
+    acc.add(own ? Sj : Si, f_S2);
+    acc.add(own ? Bi : Bj, f_B1);
+    acc.add(own ? Bj : Bi, f_B2);
+    acc.add(Bn, f_Bn);
+}
+
 } // tsp
 } // mjg

@@ -94,3 +94,28 @@ def test_mixed_small_systems_follow_fp64(system):
     rms = np.sqrt(np.mean(fa ** 2))
     print(f"[gpu] {system} mixed vs FP64: {np.sqrt(np.mean((fa - fb) ** 2)) / rms:.1e}", flush=True)
     assert np.sqrt(np.mean((fa - fb) ** 2)) < 1e-5 * rms
+
+
+@pytest.mark.parametrize("n_bp", [6, 40])
+def test_duplex_rows(n_bp):
+    """Base pairing, cross stacking (four lanes a pair) and the lists' base rules, through rebuilds."""
+    from mjolnir_amd import workloads
+    _follow(workloads.dna_duplex(n_bp, seed=4, margin=0.1), 120)
+
+
+def test_exclusions_far_apart_in_index():
+    """A hub excluded from 150 particles far from it in index: more than a rebuild keeps in LDS for a row."""
+    from mjolnir_amd.spec import GlobalSpec, IntegratorSpec, LocalSpec, SystemSpec
+    rng = np.random.default_rng(12)
+    n = 216
+    g = np.stack(np.meshgrid(*[np.arange(6)] * 3, indexing="ij"), -1).reshape(-1, 3) * 4.5
+    pos = g + rng.uniform(-0.3, 0.3, size=g.shape)
+    other = np.arange(60, 210)
+    hub = LocalSpec("BondLength", "GoContact", "contact", np.stack([np.zeros_like(other), other], 1),
+                    np.stack([np.full(len(other), 1e-3), np.full(len(other), 8.0)], 1))
+    ev = GlobalSpec(potential="ExcludedVolume", participants=np.arange(n), params=np.full((n, 1), 1.2), cutoff=2.0,
+                    epsilon=0.2, partition="CellList", margin=0.2, ignore_within={"contact": 1})
+    spec = SystemSpec(boundary="unlimited", mass=np.ones(n), pos=pos, vel=rng.normal(size=pos.shape) * 0.7,
+                      attributes={"temperature": 300.0}, local=[hub], global_=[ev],
+                      integrator=IntegratorSpec("BAOABLangevin", 0.01, np.full(n, 0.1), seed=2), name="hub")
+    _follow(spec, 120)
