@@ -462,6 +462,10 @@ void Engine::alloc_list(GlobalIA& g, uint32_t cap)
     g.cap = cap;
     g.d_nl = dalloc<uint32_t>((size_t)np * cap);
     if(g.tiled) {g.d_nl16 = dalloc<uint16_t>((size_t)np * cap);}
+    if(g.inner)
+    {
+        if(g.tiled) {g.d_in16 = dalloc<uint16_t>((size_t)np * cap);} else {g.d_in = dalloc<uint32_t>((size_t)np * cap);}
+    }
 }
 
 // The cell-tile pair kernel (tile_kernels.hpp) serves a pair interaction on a periodic cell list
@@ -626,6 +630,13 @@ void Engine::setup_global(GlobalIA& g)
             g.tile_fixed = true;
         }
     }
+    g.inner = !g.small && g.partition == MJG_PART_CELLLIST && !g.multibody() && g.margin >= kInnerMinMargin;
+    if(g.inner)
+    {
+        g.abs_inner = kInnerShare * g.margin * g.max_cutoff;
+        g.r_in = g.max_cutoff + g.abs_inner;
+        g.d_nin = dalloc<uint32_t>(np);
+    }
     g.d_nn = dalloc<uint32_t>(np);
     g.d_spart = dalloc<uint32_t>(np);
     if(g.partition == MJG_PART_CELLLIST) {g.d_spos = dalloc<double4>(np);}
@@ -684,7 +695,7 @@ ListSegTable Engine::list_table()
     return t;
 }
 
-PairSegTable Engine::pair_table(int only)
+PairSegTable Engine::pair_table(int only, bool step)
 {
     PairSegTable t{};
     uint32_t block = 0;
@@ -697,6 +708,11 @@ PairSegTable Engine::pair_table(int only)
         PairSeg& s = t.seg[t.n++];
         s.kind = g.pot;
         s.tpp = g.tpp;
+        if(step && g.inner)
+        {
+            s.tpp = g.tpp_in;
+            s.in = g.d_in; s.nin = g.d_nin; s.r_in2 = g.r_in * g.r_in; s.prune = &(d_lctl_ + gi)->prune;
+        }
         s.np = (uint32_t)g.part.size();
         s.block_begin = block;
         s.cap = g.cap;
@@ -728,6 +744,7 @@ void Engine::launch_rebuilds(int force, uint32_t k)
         ps.never_rebuild = (g.partition == MJG_PART_NAIVE);
         ps.allpairs = (g.partition != MJG_PART_CELLLIST);
         ps.abs_margin = g.max_cutoff * g.margin;
+        ps.abs_inner = g.abs_inner;
         ps.r_list = g.r_list;
         ps.part = g.d_part;
         ps.skeys = g.sb.keys;
@@ -816,6 +833,7 @@ void Engine::build_lists_now(bool)
             }
             const uint32_t t = lanes_for(ctl[g].maxcount);
             if(t != G.tpp) {G.tpp = t; again = again || false;}
+            if(G.inner) {G.tpp_in = lanes_for((uint32_t)(ctl[g].maxcount * std::pow(G.r_in / G.r_list, 3.0)));}
             uint32_t mb = 1;
             while(mb < 64 && mb < ctl[g].maxcount) {mb <<= 1;}
             G.mb_tpp = mb;
@@ -936,7 +954,8 @@ void Engine::initialize()
 
 // Every interaction's forces (local terms into their slots, pair interactions into their arrays), and
 // with `energy` the energies into h_energy_.  only >= 0 restricts the call to one interaction id.
-void Engine::interaction_forces(bool energy, int only)
+// step: a step of launch_segment, whose skin check has settled the inner lists' use.
+void Engine::interaction_forces(bool energy, int only, bool step)
 {
     const int nl = (int)locals_.size();
     const bool run_locals = local_blocks_ > 0 && (only < 0 || only < nl);
@@ -959,27 +978,31 @@ void Engine::interaction_forces(bool energy, int only)
                                d_lidx_, d_lpar_, d_tdst_, d_tf_, d_te_, only);
         }
     }
-    const PairSegTable pt = pair_table(only);
+    const PairSegTable pt = pair_table(only, step);
     if(pt.n > 0)
     {
         uint32_t blocks = 0;
         for(int k = 0; k < pt.n; ++k) {blocks += blocks_for((size_t)pt.seg[k].np * pt.seg[k].tpp, 256);}
         if(precision_ == MJG_FP32_FIXED)
         {
-            if(energy) {hipLaunchKernelGGL(k_pairs_mixed<true>, dim3(blocks), dim3(256), 0, stream_, d_pos_, box_, pt);}
-            else {hipLaunchKernelGGL(k_pairs_mixed<false>, dim3(blocks), dim3(256), 0, stream_, d_pos_, box_, pt);}
+            const dim3 grid(blocks), block(256);
+            if(energy) {hipLaunchKernelGGL((k_pairs_mixed<true, false>), grid, block, 0, stream_, d_pos_, box_, pt);}
+            else if(step) {hipLaunchKernelGGL((k_pairs_mixed<false, true>), grid, block, 0, stream_, d_pos_, box_, pt);}
+            else {hipLaunchKernelGGL((k_pairs_mixed<false, false>), grid, block, 0, stream_, d_pos_, box_, pt);}
         }
         else
         {
-            if(energy) {hipLaunchKernelGGL(k_pairs<true>, dim3(blocks), dim3(256), 0, stream_, d_pos_, box_, pt);}
-            else {hipLaunchKernelGGL(k_pairs<false>, dim3(blocks), dim3(256), 0, stream_, d_pos_, box_, pt);}
+            const dim3 grid(blocks), block(256);
+            if(energy) {hipLaunchKernelGGL((k_pairs<true, false>), grid, block, 0, stream_, d_pos_, box_, pt);}
+            else if(step) {hipLaunchKernelGGL((k_pairs<false, true>), grid, block, 0, stream_, d_pos_, box_, pt);}
+            else {hipLaunchKernelGGL((k_pairs<false, false>), grid, block, 0, stream_, d_pos_, box_, pt);}
         }
     }
     for(size_t gi = 0; gi < globals_.size(); ++gi)
     {
         if(only >= 0 && only != nl + (int)gi) {continue;}
         if(globals_[gi].multibody()) {launch_multibody(globals_[gi], energy);}
-        else if(globals_[gi].tiled) {launch_tiled(globals_[gi], (int)gi, energy);}
+        else if(globals_[gi].tiled) {launch_tiled(globals_[gi], (int)gi, energy, step);}
     }
     if(energy)
     {
@@ -1020,7 +1043,7 @@ GatherArgs Engine::gather_args(bool locals, int only, bool sums)
 // (and with `kick` applies the closing half-kick of the integrator step).
 void Engine::forces(double4* f, bool energy, int only, bool kick, bool advance)
 {
-    interaction_forces(energy, only);
+    interaction_forces(energy, only, false);
     FinishArgs fa{};
     fa.g = gather_args(local_blocks_ > 0 && (only < 0 || only < (int)locals_.size()), only, false);
     fa.halfdt = dt_ / 2;
@@ -1049,7 +1072,7 @@ void Engine::launch_multibody(const GlobalIA& g, bool energy)
 
 // Cell-tile pair kernel of one interaction: one workgroup per cell, its LDS the staging of the
 // 27-cell neighbourhood, the fused kernel's lanes per row (the same sums bit for bit).
-void Engine::launch_tiled(GlobalIA& g, int gi, bool energy)
+void Engine::launch_tiled(GlobalIA& g, int gi, bool energy, bool step)
 {
     TileSeg s{};
     PairSeg& ps = s.ps;
@@ -1061,7 +1084,9 @@ void Engine::launch_tiled(GlobalIA& g, int gi, bool energy)
     const bool mixed = (precision_ == MJG_FP32_FIXED);
     // FP64 keeps the gather kernel's lanes per row (its sums in the same order); the mixed sums are
     // exact, so its lanes per row are chosen for the tile alone
-    s.tpp = mixed ? tile_lanes(g) : g.tpp;
+    const uint32_t lanes = (step && g.inner) ? g.tpp_in : g.tpp;
+    s.tpp = mixed ? tile_lanes(lanes) : lanes;
+    if(step && g.inner) {s.in16 = g.d_in16; ps.nin = g.d_nin; ps.r_in2 = g.r_in * g.r_in;}
     const size_t lds = (size_t)g.tile_cap * (mixed ? kTileBytesPerParticleF32 : kTileBytesPerParticle);
     const dim3 grid(g.grid.ncell), block(kTileThreads);
     if(mixed)
@@ -1079,14 +1104,14 @@ void Engine::launch_tiled(GlobalIA& g, int gi, bool energy)
 // Lanes per list row of the mixed cell-tile kernel: MJG_TILE_TPP (a power of two up to 64) or half
 // the gather kernel's (about twelve entries a lane for the longest row; measured on a 262,144-particle
 // LJ fluid, 8 and 16 lanes per row ran 10 % faster than 4 or 32).
-uint32_t Engine::tile_lanes(const GlobalIA& g) const
+uint32_t Engine::tile_lanes(uint32_t gather_lanes) const
 {
     if(const char* v = std::getenv("MJG_TILE_TPP"))
     {
         const long t = std::atol(v);
         if(t >= 1 && t <= 64 && (t & (t - 1)) == 0) {return (uint32_t)t;}
     }
-    return std::max<uint32_t>(1, g.tpp / 2);
+    return std::max<uint32_t>(1, gather_lanes / 2);
 }
 
 // After lists were built: a tiled interaction whose largest neighbourhood outgrew its staging
@@ -1460,7 +1485,7 @@ void Engine::launch_step_forces(uint32_t k)
     if(!small_)
     {
         if(!globals_.empty()) {launch_rebuilds(0, k);}
-        interaction_forces(false, -1);
+        interaction_forces(false, -1, true);
         return;
     }
     SmallForces a{};
@@ -1857,7 +1882,7 @@ double Engine::profile_interaction(int id, int reps, uint64_t* half_pairs)
     const int nl = (int)locals_.size();
     uint64_t hp = 0;
     check(hipEventRecord(a, stream_), "event record");
-    const PairSegTable pt = pair_table(id);
+    const PairSegTable pt = pair_table(id, false);
     uint32_t pblocks = 0;
     for(int k = 0; k < pt.n; ++k) {pblocks += blocks_for((size_t)pt.seg[k].np * pt.seg[k].tpp, 256);}
     for(int r = 0; r < reps; ++r)
@@ -1868,14 +1893,14 @@ double Engine::profile_interaction(int id, int reps, uint64_t* half_pairs)
                                d_lidx_, d_lpar_, d_tdst_, d_tf_, d_te_, id);
         }
         else if(globals_[id - nl].multibody()) {launch_multibody(globals_[id - nl], false);}
-        else if(globals_[id - nl].tiled) {launch_tiled(globals_[id - nl], id - nl, false);}
+        else if(globals_[id - nl].tiled) {launch_tiled(globals_[id - nl], id - nl, false, false);}
         else if(precision_ == MJG_FP32_FIXED)
         {
-            hipLaunchKernelGGL(k_pairs_mixed<false>, dim3(pblocks), dim3(256), 0, stream_, d_pos_, box_, pt);
+            hipLaunchKernelGGL((k_pairs_mixed<false, false>), dim3(pblocks), dim3(256), 0, stream_, d_pos_, box_, pt);
         }
         else
         {
-            hipLaunchKernelGGL(k_pairs<false>, dim3(pblocks), dim3(256), 0, stream_, d_pos_, box_, pt);
+            hipLaunchKernelGGL((k_pairs<false, false>), dim3(pblocks), dim3(256), 0, stream_, d_pos_, box_, pt);
         }
     }
     check(hipEventRecord(b, stream_), "event record");

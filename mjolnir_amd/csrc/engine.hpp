@@ -65,6 +65,12 @@ struct GlobalIA
     double4* d_spos = nullptr;    // position of each sorted slot at the last cell-list build
     uint32_t cap = 0;             // row length of the list: nl[t * cap + k]
     uint32_t tpp = 8;             // lanes per participant in k_verlet / k_pairs
+    // inner list of a large cell list (prune_decision): its radius, margin, lanes per row and arrays
+    bool inner = false;
+    double r_in = 0, abs_inner = 0;
+    uint32_t tpp_in = 8;
+    uint32_t *d_in = nullptr, *d_nin = nullptr;
+    uint16_t* d_in16 = nullptr;
     uint32_t mb_tpp = 16;         // lanes per participant in k_tsp_pairs (one entry per lane)
     bool small = false;           // one-workgroup rebuild (np <= kSmallMaxPart)
     double* d_epair = nullptr;
@@ -148,15 +154,15 @@ class Engine
     void launch_advance(uint32_t k, bool last);
     void launch_step_forces(uint32_t k);
     void launch_segment(size_t n);
-    void interaction_forces(bool energy, int only);
+    void interaction_forces(bool energy, int only, bool step);
     void build_lists_now(bool all);
     ListSeg list_seg(GlobalIA& g, size_t gi);
     ListSegTable list_table();
-    PairSegTable pair_table(int only);
+    PairSegTable pair_table(int only, bool step);
     void launch_multibody(const GlobalIA& g, bool energy);
-    void launch_tiled(GlobalIA& g, int gi, bool energy);
+    void launch_tiled(GlobalIA& g, int gi, bool energy, bool step);
     bool grow_tiles(const std::vector<ListCtl>& ctl);
-    uint32_t tile_lanes(const GlobalIA& g) const;
+    uint32_t tile_lanes(uint32_t gather_lanes) const;
     void forces(double4* f, bool energy, int only, bool kick, bool advance = false);
     void launch_ul_accel(bool kick);
     void launch_step();

@@ -414,8 +414,26 @@ struct PairSeg
     double4* fout;
     double* eout;
     PairParams pp;
+    uint32_t* in;            // inner list of each row (as nl), its lengths, its radius squared and the
+    uint32_t* nin;           // step's choice between writing and walking it (null: no inner list)
+    double r_in2;
+    const int* prune;
 };
 constexpr int kMaxPairSegs = 16;
+// how a pair kernel uses the lists: the list as it is; the list, writing the inner one; the inner one
+enum ListUse : int {kListWhole = 0, kListPrune = 1, kListInner = 2};
+
+// The kept entries of a group's lanes (in lane order) appended to a row: `at` counts those before, and
+// the place of this lane's entry is returned.  Lanes past the end of the row are inactive here.
+__device__ __forceinline__ uint32_t group_append(bool keep, uint32_t tpp, uint32_t& at)
+{
+    const uint32_t lane = threadIdx.x % kWave;
+    const uint64_t gmask = ((tpp >= 64) ? ~0ull : ((1ull << tpp) - 1ull)) << (lane & ~(tpp - 1u));
+    const uint64_t b = __ballot(keep) & gmask;
+    const uint32_t place = at + (uint32_t)__popcll(b & ((1ull << lane) - 1ull));
+    at += (uint32_t)__popcll(b);
+    return place;
+}
 struct PairSegTable
 {
     PairSeg seg[kMaxPairSegs];
@@ -438,12 +456,13 @@ struct RowHead
     uint32_t i, cnt;
     uint32_t w[kPairBatch];
 };
+template<int USE = kListWhole>
 __device__ __forceinline__ RowHead row_head(const PairSeg& s, uint32_t t, uint32_t l)
 {
     RowHead h;
     h.i = s.spart[t];
-    h.cnt = s.nn[t];
-    const uint32_t* row = s.nl + (size_t)t * s.cap;
+    h.cnt = (USE == kListInner) ? s.nin[t] : s.nn[t];
+    const uint32_t* row = ((USE == kListInner) ? s.in : s.nl) + (size_t)t * s.cap;
 #pragma unroll
     for(int m = 0; m < kPairBatch; ++m)
     {
@@ -453,13 +472,14 @@ __device__ __forceinline__ RowHead row_head(const PairSeg& s, uint32_t t, uint32
     return h;
 }
 
-template<int KIND, bool ENERGY>
+template<int KIND, bool ENERGY, int USE = kListWhole>
 __device__ __forceinline__ void pair_row(const PairSeg& s, const RowHead& h, uint32_t t, uint32_t l,
                                          const double4* __restrict__ pos, const Box& box, double& fx, double& fy,
                                          double& fz, double& e)
 {
     const uint32_t i = h.i, cnt = h.cnt;
-    const uint32_t* row = s.nl + (size_t)t * s.cap;
+    const uint32_t* row = ((USE == kListInner) ? s.in : s.nl) + (size_t)t * s.cap;
+    uint32_t at = 0;
     uint32_t w[kPairBatch];
 #pragma unroll
     for(int m = 0; m < kPairBatch; ++m) {w[m] = h.w[m];}
@@ -492,23 +512,31 @@ __device__ __forceinline__ void pair_row(const PairSeg& s, const RowHead& h, uin
             if(k0 + m * s.tpp >= cnt) {break;}
             double dx, dy, dz;
             adjust_direction(box, ri.x, ri.y, ri.z, rj[m].x, rj[m].y, rj[m].z, dx, dy, dz);
+            if constexpr(USE == kListPrune)
+            {
+                const bool keep = length_sq(dx, dy, dz) < s.r_in2;
+                const uint32_t k = group_append(keep, s.tpp, at);
+                if(keep) {s.in[(size_t)t * s.cap + k] = j[m];}
+            }
             par.b0 = p0[m]; par.b1 = p1[m];
             pair_term_p<KIND, ENERGY>(s.pp, i, j[m], par, 0, 1, dx, dy, dz, fx, fy, fz, e);
         }
     }
+    // the group's first lane takes part in every round: it has the whole count
+    if(USE == kListPrune && l == 0) {s.nin[t] = at;}
 }
 
 // one row by the tpp lanes of a group: its force (and energy) stored by lane 0
-template<bool ENERGY>
+template<bool ENERGY, int USE = kListWhole>
 __device__ __forceinline__ void pair_row_store(const PairSeg& s, const RowHead& h, uint32_t t, uint32_t l,
                                                const double4* __restrict__ pos, const Box& box)
 {
     double fx = 0, fy = 0, fz = 0, e = 0;
     const uint32_t i = h.i;
-    if(s.kind == kPairLJ) {pair_row<kPairLJ, ENERGY>(s, h, t, l, pos, box, fx, fy, fz, e);}
-    else if(s.kind == kPairEV) {pair_row<kPairEV, ENERGY>(s, h, t, l, pos, box, fx, fy, fz, e);}
-    else if(s.kind == kPair3SPN2EV) {pair_row<kPair3SPN2EV, ENERGY>(s, h, t, l, pos, box, fx, fy, fz, e);}
-    else {pair_row<kPairDH, ENERGY>(s, h, t, l, pos, box, fx, fy, fz, e);}
+    if(s.kind == kPairLJ) {pair_row<kPairLJ, ENERGY, USE>(s, h, t, l, pos, box, fx, fy, fz, e);}
+    else if(s.kind == kPairEV) {pair_row<kPairEV, ENERGY, USE>(s, h, t, l, pos, box, fx, fy, fz, e);}
+    else if(s.kind == kPair3SPN2EV) {pair_row<kPair3SPN2EV, ENERGY, USE>(s, h, t, l, pos, box, fx, fy, fz, e);}
+    else {pair_row<kPairDH, ENERGY, USE>(s, h, t, l, pos, box, fx, fy, fz, e);}
     for(uint32_t o = s.tpp / 2; o > 0; o >>= 1)
     {
         fx += __shfl_xor(fx, o, kWave);
@@ -523,7 +551,8 @@ __device__ __forceinline__ void pair_row_store(const PairSeg& s, const RowHead& 
     }
 }
 
-template<bool ENERGY>
+// STEP: inside an integrator step, where interactions with an inner list use it
+template<bool ENERGY, bool STEP>
 __global__ void __launch_bounds__(256)
 k_pairs(const double4* __restrict__ pos, Box box, PairSegTable tab)
 {
@@ -533,6 +562,15 @@ k_pairs(const double4* __restrict__ pos, Box box, PairSegTable tab)
     const uint32_t gt = (blockIdx.x - s.block_begin) * blockDim.x + threadIdx.x;
     const uint32_t t = gt / s.tpp, l = gt % s.tpp;
     if(t >= s.np) {return;}   // whole groups leave together
+    if constexpr(STEP)
+    {
+        if(s.in != nullptr)
+        {
+            if(*s.prune) {pair_row_store<ENERGY, kListPrune>(s, row_head(s, t, l), t, l, pos, box);}
+            else {pair_row_store<ENERGY, kListInner>(s, row_head<kListInner>(s, t, l), t, l, pos, box);}
+            return;
+        }
+    }
     pair_row_store<ENERGY>(s, row_head(s, t, l), t, l, pos, box);
 }
 
@@ -623,14 +661,15 @@ __device__ __forceinline__ bool pair_term_f32(const PairConstsF& K, const PairPa
     return true;
 }
 
-template<int KIND, bool ENERGY>
+template<int KIND, bool ENERGY, int USE = kListWhole>
 __device__ __forceinline__ void pair_row_mixed(const PairSeg& s, const RowHead& h, uint32_t t, uint32_t l,
                                                const double4* __restrict__ pos, const Box& box, long long& ax,
                                                long long& ay, long long& az, double& e)
 {
     const PairConstsF K = pair_consts_f(s.pp);
     const uint32_t i = h.i, cnt = h.cnt;
-    const uint32_t* row = s.nl + (size_t)t * s.cap;
+    const uint32_t* row = ((USE == kListInner) ? s.in : s.nl) + (size_t)t * s.cap;
+    uint32_t at = 0;
     uint32_t w[kPairBatch];
 #pragma unroll
     for(int m = 0; m < kPairBatch; ++m) {w[m] = h.w[m];}
@@ -663,6 +702,12 @@ __device__ __forceinline__ void pair_row_mixed(const PairSeg& s, const RowHead& 
             if(k0 + m * s.tpp >= cnt) {break;}
             double ddx, ddy, ddz;
             adjust_direction(box, ri.x, ri.y, ri.z, rj[m].x, rj[m].y, rj[m].z, ddx, ddy, ddz);
+            if constexpr(USE == kListPrune)
+            {
+                const bool keep = length_sq(ddx, ddy, ddz) < s.r_in2;
+                const uint32_t k = group_append(keep, s.tpp, at);
+                if(keep) {s.in[(size_t)t * s.cap + k] = j[m];}
+            }
             par.b0 = p0[m]; par.b1 = p1[m];
             float c;
             if(!pair_term_f32<KIND, ENERGY>(K, s.pp, par, i, j[m], 0, 1, ddx, ddy, ddz, c, e)) {continue;}
@@ -672,6 +717,8 @@ __device__ __forceinline__ void pair_row_mixed(const PairSeg& s, const RowHead& 
             ax += fx; ay += fy; az += fz;
         }
     }
+    // the group's first lane takes part in every round: it has the whole count
+    if(USE == kListPrune && l == 0) {s.nin[t] = at;}
 }
 
 __device__ __forceinline__ long long shfl_xor_ll(long long v, int o)
@@ -680,17 +727,17 @@ __device__ __forceinline__ long long shfl_xor_ll(long long v, int o)
     return ((long long)hi << 32) | (unsigned int)lo;
 }
 
-template<bool ENERGY>
+template<bool ENERGY, int USE = kListWhole>
 __device__ __forceinline__ void pair_row_mixed_store(const PairSeg& s, const RowHead& h, uint32_t t, uint32_t l,
                                                      const double4* __restrict__ pos, const Box& box)
 {
     long long ax = 0, ay = 0, az = 0;
     double e = 0;
     const uint32_t i = h.i;
-    if(s.kind == kPairLJ) {pair_row_mixed<kPairLJ, ENERGY>(s, h, t, l, pos, box, ax, ay, az, e);}
-    else if(s.kind == kPairEV) {pair_row_mixed<kPairEV, ENERGY>(s, h, t, l, pos, box, ax, ay, az, e);}
-    else if(s.kind == kPair3SPN2EV) {pair_row_mixed<kPair3SPN2EV, ENERGY>(s, h, t, l, pos, box, ax, ay, az, e);}
-    else {pair_row_mixed<kPairDH, ENERGY>(s, h, t, l, pos, box, ax, ay, az, e);}
+    if(s.kind == kPairLJ) {pair_row_mixed<kPairLJ, ENERGY, USE>(s, h, t, l, pos, box, ax, ay, az, e);}
+    else if(s.kind == kPairEV) {pair_row_mixed<kPairEV, ENERGY, USE>(s, h, t, l, pos, box, ax, ay, az, e);}
+    else if(s.kind == kPair3SPN2EV) {pair_row_mixed<kPair3SPN2EV, ENERGY, USE>(s, h, t, l, pos, box, ax, ay, az, e);}
+    else {pair_row_mixed<kPairDH, ENERGY, USE>(s, h, t, l, pos, box, ax, ay, az, e);}
     for(uint32_t o = s.tpp / 2; o > 0; o >>= 1)
     {
         ax += shfl_xor_ll(ax, (int)o);
@@ -709,7 +756,8 @@ __device__ __forceinline__ void pair_row_mixed_store(const PairSeg& s, const Row
     }
 }
 
-template<bool ENERGY>
+// STEP: inside an integrator step, where interactions with an inner list use it
+template<bool ENERGY, bool STEP>
 __global__ void __launch_bounds__(256)
 k_pairs_mixed(const double4* __restrict__ pos, Box box, PairSegTable tab)
 {
@@ -719,6 +767,15 @@ k_pairs_mixed(const double4* __restrict__ pos, Box box, PairSegTable tab)
     const uint32_t gt = (blockIdx.x - s.block_begin) * blockDim.x + threadIdx.x;
     const uint32_t t = gt / s.tpp, l = gt % s.tpp;
     if(t >= s.np) {return;}   // whole groups leave together
+    if constexpr(STEP)
+    {
+        if(s.in != nullptr)
+        {
+            if(*s.prune) {pair_row_mixed_store<ENERGY, kListPrune>(s, row_head(s, t, l), t, l, pos, box);}
+            else {pair_row_mixed_store<ENERGY, kListInner>(s, row_head<kListInner>(s, t, l), t, l, pos, box);}
+            return;
+        }
+    }
     pair_row_mixed_store<ENERGY>(s, row_head(s, t, l), t, l, pos, box);
 }
 

@@ -53,7 +53,28 @@ struct ListCtl
     unsigned long long bbox_min[3];
     unsigned long long bbox_max[3];
     double margin;                 // current_margin of the partition
+    double inner;                  // margin left of the inner list (prune_decision)
+    int prune;                     // 1: this step's pair kernel writes the inner list, 0: it walks it
 };
+
+// Inner lists.  The list radius r_c (1 + m) is the reference's (its pairs, its rebuild steps), and with
+// the input's usual m = 0.5 a row holds 3.4 times the partners inside the cutoff.  Between rebuilds the
+// pair kernels of the large interactions therefore walk an inner list, the row's entries within
+// r_c + kInnerShare m r_c in their order, written by the pair kernel itself on the first step of a
+// segment, after a rebuild and whenever the displacements since have used up the inner margin.  A
+// pair inside the cutoff is never missed (the inner margin is spent as the outer one is), so the
+// forces are the same sums.  A row walked costs (1 + x m)^3 entries plus (1 + m)^3 / (x K) for its
+// share of the walk that writes it, K the steps between rebuilds (about 60 for a fluid at m = 0.5):
+// flat around x = 0.2, 1.6 against 3.4, and 1.5 against 1.7 at m = 0.2, below which there are none.
+constexpr double kInnerShare = 0.2;
+constexpr double kInnerMinMargin = 0.2;
+__device__ __forceinline__ void prune_decision(ListCtl& c, double dmargin, double abs_inner, uint32_t k)
+{
+    const double m = c.inner - dmargin;
+    const bool p = k == 0 || c.rebuild != 0 || !(m >= 0);
+    c.inner = p ? abs_inner : m;
+    c.prune = p ? 1 : 0;
+}
 
 // ForceField::reduce_margin (ForceField.hpp:75-92) called from the host: every list's margin less
 // dmargin; *spent (pinned host memory) tells whether one ran out.  One thread per interaction of a
@@ -570,6 +591,7 @@ struct PrepSeg
     int never_rebuild;       // Naive partition
     int allpairs;            // Verlet / Naive: no cells to prepare
     double abs_margin;       // cutoff * margin
+    double abs_inner;        // margin of the inner list (0: none is kept)
     double r_list;
     const uint32_t* part;
     uint32_t* skeys;
@@ -743,6 +765,7 @@ __global__ void k_margin_large(PrepSegTable tab, StepCtl* __restrict__ sctl, uin
         const PrepSeg& s = tab.seg[g];
         const double dmargin = 2 * sqrt(__longlong_as_double((long long)sctl->maxdisp2[(sctl->step + k) & 1]));
         if(margin_decision(*s.ctl, dmargin, s.abs_margin, s.never_rebuild, force)) {atomicAdd(&sctl->rebuilds, 1ull);}
+        prune_decision(*s.ctl, dmargin, s.abs_inner, force ? 0u : k);
     }
 }
 

@@ -18,6 +18,8 @@
 #include "force_kernels.hpp"
 #include "nlist_kernels.hpp"
 
+#include <type_traits>
+
 namespace mjg
 {
 struct TileSeg
@@ -31,6 +33,8 @@ struct TileSeg
     const ListCtl* ctl;
     uint32_t cap_nbr;             // staging capacity in particles
     uint32_t tpp;                 // lanes per row of this kernel
+    uint16_t* in16;               // staging slots of the inner list's entries (null: no inner list in
+                                  // this launch); rows served from global memory walk the whole list
 };
 constexpr uint32_t kTileThreads = 256;
 constexpr int kTileBatch = 4;
@@ -48,7 +52,16 @@ constexpr size_t kTileBytesPerParticle = 5 * sizeof(double) + sizeof(uint32_t);
 // staged particles per thread whose loads are issued together
 constexpr int kTileStage = 4;
 
-template<bool MIXED, bool ENERGY, int KIND>
+// the launch's use of the lists (uniform: one word); an energy call walks the whole list
+template<bool ENERGY, typename F>
+__device__ __forceinline__ void tile_use(const TileSeg& s, F&& rows)
+{
+    if(ENERGY || s.in16 == nullptr) {rows(std::integral_constant<int, kListWhole>{});}
+    else if(s.ctl->prune) {rows(std::integral_constant<int, kListPrune>{});}
+    else {rows(std::integral_constant<int, kListInner>{});}
+}
+
+template<bool MIXED, bool ENERGY, int KIND, int USE>
 __device__ __forceinline__ void tile_rows(const TileSeg& s, const Box& box, uint32_t cs, uint32_t nhome, uint32_t home0,
                                           const double* sx, const double* sy, const double* sz, const StagePar& par,
                                           const uint32_t* sid)
@@ -63,8 +76,9 @@ __device__ __forceinline__ void tile_rows(const TileSeg& s, const Box& box, uint
         const uint32_t t = cs + h, ki = home0 + h;
         const uint32_t i = sid[ki];
         const double xi = sx[ki], yi = sy[ki], zi = sz[ki];
-        const uint32_t cnt = ps.nn[t];
-        const uint16_t* row = s.nl16 + (size_t)t * ps.cap;
+        const uint32_t cnt = (USE == kListInner) ? ps.nin[t] : ps.nn[t];
+        const uint16_t* row = ((USE == kListInner) ? (const uint16_t*)s.in16 : s.nl16) + (size_t)t * ps.cap;
+        uint32_t at = 0;
         double fx = 0, fy = 0, fz = 0, e = 0;
         long long ax = 0, ay = 0, az = 0;
         // the entries k = l, l + tpp, ... in order, kTileBatch at a time: a batch's row words come
@@ -91,6 +105,12 @@ __device__ __forceinline__ void tile_rows(const TileSeg& s, const Box& box, uint
                 const uint32_t j = sid[kj[m]];
                 double dx, dy, dz;
                 adjust_direction(box, xi, yi, zi, sx[kj[m]], sy[kj[m]], sz[kj[m]], dx, dy, dz);
+                if constexpr(USE == kListPrune)
+                {
+                    const bool keep = length_sq(dx, dy, dz) < ps.r_in2;
+                    const uint32_t k = group_append(keep, tpp, at);
+                    if(keep) {s.in16[(size_t)t * ps.cap + k] = (uint16_t)kj[m];}
+                }
                 if constexpr(MIXED)
                 {
                     float c;
@@ -123,6 +143,7 @@ __device__ __forceinline__ void tile_rows(const TileSeg& s, const Box& box, uint
         }
         if(l == 0)
         {
+            if(USE == kListPrune) {ps.nin[t] = at;}
             if constexpr(MIXED)
             {
                 const bool bad = fix_insane((unsigned long long)ax) || fix_insane((unsigned long long)ay) ||
@@ -290,7 +311,10 @@ __device__ __forceinline__ void tile_cell(const TileSeg& s, const double4* __res
         }
     }
     __syncthreads();
-    tile_rows<MIXED, ENERGY, KIND>(s, box, cs, nhome, c_off[13], sx, sy, sz, StagePar{s0, s1}, sid);
+    auto rows = [&](auto use) {
+        tile_rows<MIXED, ENERGY, KIND, decltype(use)::value>(s, box, cs, nhome, c_off[13], sx, sy, sz, StagePar{s0, s1}, sid);
+    };
+    tile_use<ENERGY>(s, rows);
 }
 
 // ------------------------------------------------------------------------------------
@@ -345,7 +369,7 @@ __device__ __forceinline__ uint32_t tile_slot_particle(const TileSeg& s, const u
     return s.spart[c_beg[m] + (k - c_off[m])];
 }
 
-template<bool ENERGY, int KIND>
+template<bool ENERGY, int KIND, int USE>
 __device__ __forceinline__ void tile_rows_f32(const TileSeg& s, const double4* __restrict__ pos, const Box& box,
                                               uint32_t cs, uint32_t nhome, uint32_t home0, const float4* hi,
                                               const float4* lo, const uint32_t* c_beg, const uint32_t* c_off)
@@ -356,14 +380,16 @@ __device__ __forceinline__ void tile_rows_f32(const TileSeg& s, const double4* _
     const uint32_t tid = threadIdx.x;
     const PairConstsF K = pair_consts_f(ps.pp);
     const float acut2 = (float)(ps.pp.abs_cutoff * ps.pp.abs_cutoff);
+    const float rin2 = (float)ps.r_in2 * (1.0f + kTileBand);
     for(uint32_t u = tid; u < nhome * tpp; u += kTileThreads)
     {
         const uint32_t h = u / tpp, l = u % tpp;
         const uint32_t t = cs + h, ki = home0 + h;
         const uint32_t i = s.spart[t];
         const float4 ah = hi[ki], al = lo[ki];
-        const uint32_t cnt = ps.nn[t];
-        const uint16_t* row = s.nl16 + (size_t)t * ps.cap;
+        const uint32_t cnt = (USE == kListInner) ? ps.nin[t] : ps.nn[t];
+        const uint16_t* row = ((USE == kListInner) ? (const uint16_t*)s.in16 : s.nl16) + (size_t)t * ps.cap;
+        uint32_t at = 0;
         double e = 0;
         long long ax = 0, ay = 0, az = 0;
         constexpr int B = kTileBatch;
@@ -390,6 +416,12 @@ __device__ __forceinline__ void tile_rows_f32(const TileSeg& s, const double4* _
                 const float dy = (bh.y - ah.y) + (bl.y - al.y);
                 const float dz = (bh.z - ah.z) + (bl.z - al.z);
                 const float l_sq = dx * dx + dy * dy + dz * dz;
+                if constexpr(USE == kListPrune)
+                {
+                    const bool keep = l_sq < rin2;
+                    const uint32_t k = group_append(keep, tpp, at);
+                    if(keep) {s.in16[(size_t)t * ps.cap + k] = (uint16_t)kj[m];}
+                }
                 float thr, sg = 0.0f;
                 if(KIND == kPairLJ) {sg = (ah.w + bh.w) * 0.5f; thr = sg * sg * K.cut2;}
                 else if(KIND == kPairEV) {sg = ah.w + bh.w; thr = sg * sg * K.cut2;}
@@ -457,6 +489,7 @@ __device__ __forceinline__ void tile_rows_f32(const TileSeg& s, const double4* _
         }
         if(l == 0)
         {
+            if(USE == kListPrune) {ps.nin[t] = at;}
             const bool bad = fix_insane((unsigned long long)ax) || fix_insane((unsigned long long)ay) ||
                              fix_insane((unsigned long long)az);
             const double nan = bad ? __builtin_nan("") : 0.0;
@@ -536,7 +569,10 @@ __device__ __forceinline__ void tile_cell_f32(const TileSeg& s, const double4* _
         }
     }
     __syncthreads();
-    tile_rows_f32<ENERGY, KIND>(s, pos, box, cs, nhome, c_off[13], hi, lo, c_beg, c_off);
+    auto rows = [&](auto use) {
+        tile_rows_f32<ENERGY, KIND, decltype(use)::value>(s, pos, box, cs, nhome, c_off[13], hi, lo, c_beg, c_off);
+    };
+    tile_use<ENERGY>(s, rows);
 }
 
 // ------------------------------------------------------------------------------------

@@ -44,10 +44,12 @@ def _gjf(spec):
     return dataclasses.replace(spec, integrator=it)
 
 
-@pytest.mark.parametrize("n,steps", [(65, 150), (257, 150), (1000, 150), (4096, 70), (4097, 70)])
-def test_fluids_at_the_edges_of_the_size_rule(n, steps):
+@pytest.mark.parametrize("n,steps,margin", [(65, 150, 0.15), (257, 150, 0.15), (1000, 150, 0.5), (4096, 70, 0.5),
+                                            (4097, 70, 0.5), (4200, 70, 0.19), (4200, 70, 0.2)])
+def test_fluids_at_the_edges_of_the_size_rule(n, steps, margin):
+    """Lists kept by the force kernel up to 4096 participants; above, inner lists from a margin of 0.2 on."""
     from mjolnir_amd import workloads
-    spec = workloads.lj_fluid(n=n, seed=n, margin=0.15 if n < 300 else 0.5)
+    spec = workloads.lj_fluid(n=n, seed=n, margin=margin)
     e = _follow(spec, steps)
     assert e.counters()[1] >= 1
 
