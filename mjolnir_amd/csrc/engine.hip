@@ -473,7 +473,7 @@ void Engine::alloc_list(GlobalIA& g, uint32_t cap)
 // kernel off): it needs a launch of one workgroup per cell, which fills the GPU only for large
 // grids.  Its staging capacity starts at twice the mean 27-cell neighbourhood and grows with the
 // largest one a build reports (ListCtl::maxnbr), up to what the LDS of one workgroup holds after
-// the kernel's static LDS (896 bytes in the current build; 4 KiB are set aside for it).
+// the kernel's static LDS (224 bytes in the current build; 4 KiB are set aside for it).
 constexpr uint32_t kTileMinNp = 16384;
 constexpr uint32_t kTileMaxCap = (uint32_t)((160 * 1024 - 4096) / kTileBytesPerParticle);
 static uint32_t tile_min_np()
@@ -481,6 +481,10 @@ static uint32_t tile_min_np()
     if(const char* v = std::getenv("MJG_TILE_MIN_NP")) {return (uint32_t)std::max(0L, std::atol(v));}
     return kTileMinNp;
 }
+
+// Blocks of the sort kernels at most: a step without a rebuild launches them all the same, and 1024
+// blocks that leave at once take about 2 us longer than 256.
+constexpr uint32_t kSortBlocks = 256;
 
 // Largest interaction whose list k_forces keeps by brute force (np^2 / 2 distance tests a rebuild).
 constexpr size_t kSelfMaxPart = 4096;
@@ -621,6 +625,11 @@ void Engine::setup_global(GlobalIA& g)
     if(g.tiled)
     {
         const double mean_nbr = 27.0 * (double)np / (double)g.grid.ncell;
+        g.fast_build = true;
+        for(int d = 0; d < 3; ++d)
+        {
+            g.fast_build = g.fast_build && (g.grid.dim[d] - 2) * (box_.width[d] / g.grid.dim[d]) >= g.r_list;
+        }
         g.tile_cap = (uint32_t)std::min<double>(kTileMaxCap, std::max(256.0, 1.25 * mean_nbr + 64.0));
         // MJG_TILE_CAP fixes the staging capacity (no growth): a capacity below the largest
         // neighbourhood serves every build from global memory
@@ -639,6 +648,7 @@ void Engine::setup_global(GlobalIA& g)
     }
     g.d_nn = dalloc<uint32_t>(np);
     g.d_spart = dalloc<uint32_t>(np);
+    if(g.tiled) {g.d_slots = dalloc<TileSlot<false>>(np);}
     if(g.partition == MJG_PART_CELLLIST) {g.d_spos = dalloc<double4>(np);}
     g.d_epair = dalloc<double>(np);
     g.d_fg = dalloc<double4>(n_);
@@ -646,7 +656,16 @@ void Engine::setup_global(GlobalIA& g)
     if(g.multibody()) {g.d_acc = dalloc<unsigned long long>(3 * n_ + 1);}   // sums and the flag word
     sync();
     g.tpp = 8;
-    alloc_list(g, 64);
+    // the first row length: a quarter above the mean of a periodic cell list (a liquid's longest row), so
+    // that its first build is kept; grown where a row is longer
+    uint32_t cap = 64;
+    if(box_.periodic && g.partition == MJG_PART_CELLLIST)
+    {
+        const double volume = box_.width[0] * box_.width[1] * box_.width[2];
+        const double mean = (double)np * (4.0 / 3.0 * 3.14159265358979323846) * g.r_list * g.r_list * g.r_list / volume;
+        cap = std::max<uint32_t>(cap, (uint32_t)std::min<double>((double)np, 1.3 * mean + 24.0));
+    }
+    alloc_list(g, cap);
 }
 
 ListSeg Engine::list_seg(GlobalIA& g, size_t gi)
@@ -776,13 +795,13 @@ void Engine::launch_rebuilds(int force, uint32_t k)
             }
             // a periodic grid's cell count is known here; an open grid's is set on the device
             const uint32_t cells = box_.periodic ? g.grid.ncell : kMaxCells;
-            hipLaunchKernelGGL(k_cellkey, dim3(blocks_for(np, 256)), dim3(256), 0, stream_, d_pos_, g.d_part, np,
+            hipLaunchKernelGGL(k_cellkey, dim3(std::min(blocks_for(np, 256), kSortBlocks)), dim3(256), 0, stream_, d_pos_, g.d_part, np,
                                g.d_grid, g.sb.ukeys, g.sb.count, ctl);
             hipLaunchKernelGGL(k_cell_scan, dim3(1), dim3(1024), 0, stream_, g.d_grid, g.sb.count, g.d_cell_start,
                                g.d_cell_end, ctl);
-            hipLaunchKernelGGL(k_cell_place, dim3(blocks_for(np, 256)), dim3(256), 0, stream_, g.sb.ukeys, np,
+            hipLaunchKernelGGL(k_cell_place, dim3(std::min(blocks_for(np, 256), kSortBlocks)), dim3(256), 0, stream_, g.sb.ukeys, np,
                                g.d_cell_end, g.sb.keys, g.sb.vals, ctl);
-            hipLaunchKernelGGL(k_cell_order, dim3(std::min<uint32_t>(blocks_for(cells, 256), 1024)), dim3(256), 0,
+            hipLaunchKernelGGL(k_cell_order, dim3(std::min(blocks_for(cells, 256 / kWave), kSortBlocks)), dim3(256), 0,
                                stream_, g.d_grid, g.d_cell_start, g.d_cell_end, g.sb.count, g.sb.vals, d_pos_,
                                g.d_part, g.d_spart, g.d_spos, ctl);
         }
@@ -805,9 +824,17 @@ void Engine::launch_rebuilds(int force, uint32_t k)
         GlobalIA& g = globals_[gi];
         if(!g.tiled) {continue;}
         const ListSeg s = list_seg(g, gi);
-        const size_t lds = (size_t)g.tile_cap * kBuildBytesPerParticle;
-        hipLaunchKernelGGL(k_verlet_tiled, dim3(std::min<uint32_t>(g.grid.ncell, kVerletMaxBlocks)), dim3(kTileThreads),
-                           lds, stream_, d_pos_, box_, s, g.tile_cap);
+        const uint32_t blocks = std::min<uint32_t>(blocks_for(g.grid.ncell, kXcds) * kXcds, kVerletMaxBlocks);
+        if(g.fast_build)
+        {
+            hipLaunchKernelGGL(k_verlet_tiled<true>, dim3(blocks), dim3(kTileThreads),
+                               (size_t)g.tile_cap * kBuildBytesPerParticleF32, stream_, d_pos_, box_, s, g.tile_cap);
+        }
+        else
+        {
+            hipLaunchKernelGGL(k_verlet_tiled<false>, dim3(blocks), dim3(kTileThreads),
+                               (size_t)g.tile_cap * kBuildBytesPerParticle, stream_, d_pos_, box_, s, g.tile_cap);
+        }
     }
 }
 
@@ -855,15 +882,20 @@ void Engine::initialize()
     if(initialized_) {throw std::invalid_argument("force field already initialized");}
     // the cell-tile kernel stages up to kTileMaxCap particles in the LDS of one workgroup
     const int tile_lds = (int)((size_t)kTileMaxCap * kTileBytesPerParticle);
-    check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pairs_tiled<true, true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, tile_lds), "tile attribute");
-    check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pairs_tiled<true, false>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, tile_lds), "tile attribute");
-    check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pairs_tiled<false, true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, tile_lds), "tile attribute");
-    check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pairs_tiled<false, false>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, tile_lds), "tile attribute");
-    check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_verlet_tiled), hipFuncAttributeMaxDynamicSharedMemorySize,
+    for(const auto& g : globals_)
+    {
+        if(g.multibody()) {continue;}
+        for(bool energy : {false, true})
+        {
+            check(hipFuncSetAttribute(reinterpret_cast<const void*>(tile_kernel(precision_ == MJG_FP32_FIXED, energy, g.pot)),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, tile_lds), "tile attribute");
+        }
+    }
+    check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_verlet_tiled<true>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)((size_t)kTileMaxCap * kBuildBytesPerParticleF32)), "tile attribute");
+    check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_verlet_tiled<false>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)((size_t)kTileMaxCap * kBuildBytesPerParticle)), "tile attribute");
     write_topology();
 
@@ -1080,7 +1112,13 @@ void Engine::launch_tiled(GlobalIA& g, int gi, bool energy, bool step)
     ps.spart = g.d_spart; ps.nl = g.d_nl; ps.nn = g.d_nn; ps.ppar = g.d_ppar;
     ps.fout = g.d_fg; ps.eout = g.d_epair; ps.pp = g.pp;
     s.nl16 = g.d_nl16; s.spart = g.d_spart; s.cell_start = g.d_cell_start; s.cell_end = g.d_cell_end;
-    s.grid = g.d_grid; s.ctl = d_lctl_ + gi; s.cap_nbr = g.tile_cap;
+    s.grid = g.grid; s.ctl = d_lctl_ + gi; s.cap_nbr = g.tile_cap;
+    for(int d = 0; d < 3; ++d)
+    {
+        const double w = box_.width[d] / g.grid.dim[d];
+        s.wh[d] = (float)w;
+        s.wl[d] = (float)(w - (double)s.wh[d]);
+    }
     const bool mixed = (precision_ == MJG_FP32_FIXED);
     // FP64 keeps the gather kernel's lanes per row (its sums in the same order); the mixed sums are
     // exact, so its lanes per row are chosen for the tile alone
@@ -1088,17 +1126,20 @@ void Engine::launch_tiled(GlobalIA& g, int gi, bool energy, bool step)
     s.tpp = mixed ? tile_lanes(lanes) : lanes;
     if(step && g.inner) {s.in16 = g.d_in16; ps.nin = g.d_nin; ps.r_in2 = g.r_in * g.r_in;}
     const size_t lds = (size_t)g.tile_cap * (mixed ? kTileBytesPerParticleF32 : kTileBytesPerParticle);
-    const dim3 grid(g.grid.ncell), block(kTileThreads);
+    s.slots = g.d_slots;
+    const dim3 slot_blocks(blocks_for(ps.np, 256));
     if(mixed)
     {
-        if(energy) {hipLaunchKernelGGL((k_pairs_tiled<true, true>), grid, block, lds, stream_, d_pos_, box_, s);}
-        else {hipLaunchKernelGGL((k_pairs_tiled<true, false>), grid, block, lds, stream_, d_pos_, box_, s);}
+        hipLaunchKernelGGL(k_tile_slots<true>, slot_blocks, dim3(256), 0, stream_, d_pos_, box_, g.d_spart, g.sb.keys,
+                           g.d_grid, g.d_ppar, g.npar, ps.np, g.d_slots);
     }
     else
     {
-        if(energy) {hipLaunchKernelGGL((k_pairs_tiled<false, true>), grid, block, lds, stream_, d_pos_, box_, s);}
-        else {hipLaunchKernelGGL((k_pairs_tiled<false, false>), grid, block, lds, stream_, d_pos_, box_, s);}
+        hipLaunchKernelGGL(k_tile_slots<false>, slot_blocks, dim3(256), 0, stream_, d_pos_, box_, g.d_spart, g.sb.keys,
+                           g.d_grid, g.d_ppar, g.npar, ps.np, g.d_slots);
     }
+    hipLaunchKernelGGL(tile_kernel(mixed, energy, g.pot), dim3(blocks_for(g.grid.ncell, kXcds) * kXcds), dim3(kTileThreads), lds, stream_, d_pos_,
+                       box_, s);
 }
 
 // Lanes per list row of the mixed cell-tile kernel: MJG_TILE_TPP (a power of two up to 64) or half

@@ -80,8 +80,10 @@ struct GlobalIA
     // staging capacity in particles
     bool tiled = false;
     uint16_t* d_nl16 = nullptr;
+    void* d_slots = nullptr;  // positions and parameters in slot order (k_tile_slots)
     uint32_t tile_cap = 0;
     bool tile_fixed = false;
+    bool fast_build = false;      // the grid allows the FP32 tests of k_verlet_tiled
     bool multibody() const {return pot == kBasePair || pot == kCrossStack;}
 };
 
