@@ -9,7 +9,15 @@ type, energy flag and 3SPN2 flag (``batch_seg.hip``).  Flags:
 * ``-ffp-contract=off``: no fused multiply-add contraction, so distance tests and FP64 forces
   follow the reference's operation order (the FP32 replica-kernel units allow contraction: they
   are held to the mixed-precision force bar, and their distance tests keep the FP64 order);
-* ``-Xclang -target-feature -Xclang -packed-fp32-ops``: no packed FP32 instructions.
+* ``-Xclang -target-feature -Xclang -packed-fp32-ops``: no packed FP32 instructions;
+* ``-disable-machine-licm`` (replica-kernel units): no code motion out of loops after instruction
+  selection.  A segment's step loop holds every term of the force field, and the code generator
+  would keep all of their literals (the coefficients of acos, exp, sin ...) in registers across
+  it: with the 3SPN2 terms that took 229-386 spilled registers and 552-600 bytes of scratch per
+  lane at 1024 threads, reloaded where each term needs them.  A literal made where it is used costs
+  one scalar move.  96 mixed-precision duplexes: 86.3 -> 49.2 us a step; the same results bit for
+  bit.  The chains, which spilled nothing, and the single-system kernels, which have no such
+  loop, measured within 1 % either way, and the single-system kernels are built without it.
 """
 from __future__ import annotations
 
@@ -29,6 +37,8 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
+NO_HOIST = ["-Xarch_device", "-mllvm=-disable-machine-licm"]
+
 
 def units():
     """(object name, source, extra flags) of every translation unit."""
@@ -41,7 +51,7 @@ def units():
         for energy in (0, 1):
             for tsp in (0, 1):
                 out.append((f"batch_seg_{real}_e{energy}_t{tsp}", "batch_seg.hip",
-                            [f"-DMJG_SEG_REAL={real}", f"-DMJG_SEG_ENERGY={energy}", f"-DMJG_SEG_TSP={tsp}"] + contract))
+                            [f"-DMJG_SEG_REAL={real}", f"-DMJG_SEG_ENERGY={energy}", f"-DMJG_SEG_TSP={tsp}"] + contract + NO_HOIST))
     return out
 
 

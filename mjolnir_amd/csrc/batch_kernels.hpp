@@ -1392,6 +1392,11 @@ __device__ __forceinline__ void rep_segment(const RepDesc& R, int nsteps, int ev
         __syncthreads();
         if(s_any_rebuild)
         {
+            // The list builds are calls that take the box and the positions by reference: they get
+            // copies of their own, so that the ones every displacement of a step reads stay in
+            // registers (with their address taken, both lived in scratch memory).
+            const Box build_box = box;
+            const PosL build_pos = P;
             for(int g = 0; g < ng; ++g)
             {
                 if(!s_rebuild[g]) {continue;}
@@ -1399,10 +1404,10 @@ __device__ __forceinline__ void rep_segment(const RepDesc& R, int nsteps, int ev
                 if(G.use_distance && G.np > kGridMinNp)
                 {
                     // the grid build synchronizes internally; the condition is uniform
-                    rep_build_grid<BS>(G, R, box, P, part_lds + G.part_off, grid_end, grid_key, grid_sorted, &s_count[g]);
+                    rep_build_grid<BS>(G, R, build_box, build_pos, part_lds + G.part_off, grid_end, grid_key, grid_sorted, &s_count[g]);
                     __syncthreads();
                 }
-                else {rep_build_rows<BS>(G, R, box, P, part_lds + G.part_off, &s_count[g]);}
+                else {rep_build_rows<BS>(G, R, build_box, build_pos, part_lds + G.part_off, &s_count[g]);}
             }
             __syncthreads();
             if(tid == 0)
