@@ -51,7 +51,8 @@ def units():
         for energy in (0, 1):
             for tsp in (0, 1):
                 out.append((f"batch_seg_{real}_e{energy}_t{tsp}", "batch_seg.hip",
-                            [f"-DMJG_SEG_REAL={real}", f"-DMJG_SEG_ENERGY={energy}", f"-DMJG_SEG_TSP={tsp}"] + contract + NO_HOIST))
+                            [f"-DMJG_SEG_REAL={real}", f"-DMJG_SEG_ENERGY={energy}", f"-DMJG_SEG_TSP={tsp}"]
+                            + (["-DMJG_SEG_WIDE"] if (real, energy, tsp) == ("double", 0, 0) else []) + contract + NO_HOIST))
     return out
 
 

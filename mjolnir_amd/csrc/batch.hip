@@ -136,6 +136,9 @@ class Batch
         if(const char* a = std::getenv("MJG_AUTOTUNE")) {autotune_ = a[0] != '0';}
         set_lds_limits<float>();
         set_lds_limits<double>();
+        int dev = 0;
+        hip_check(hipGetDevice(&dev), "hipGetDevice");
+        hip_check(hipDeviceGetAttribute(&n_cu_, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute");
         if(transfer_.create(kRepMaxN) != hipSuccess) {throw std::bad_alloc();}
     }
     ~Batch()
@@ -1066,22 +1069,20 @@ class Batch
     static uint32_t grown_cap(uint32_t seen) {return seen + seen / 2 + 1024;}
     static constexpr uint64_t kRepAllPairsMax = uint64_t(1) << 21;
 
-    template<typename Real, bool ENERGY, int BS, int PPT>
+    template<typename Real, bool ENERGY, int C, bool TSP>
     void set_lds_limit()
     {
-        hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_replica_segment<Real, ENERGY, BS, PPT, false>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRepLdsLimit),
-                  "LDS attribute");
-        hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_replica_segment<Real, ENERGY, BS, PPT, true>),
+        hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(&MJG_REP_KERNEL(Real, ENERGY, C, TSP)),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRepLdsLimit),
                   "LDS attribute");
     }
-    template<typename Real, int C> using Shape = RepShape<Real, C>;
     template<typename Real, int C>
     void set_lds_limits_class()
     {
-        set_lds_limit<Real, false, Shape<Real, C>::bs, Shape<Real, C>::ppt>();
-        set_lds_limit<Real, true, Shape<Real, C>::bs, Shape<Real, C>::ppt>();
+        set_lds_limit<Real, false, C, false>();
+        set_lds_limit<Real, false, C, true>();
+        set_lds_limit<Real, true, C, false>();
+        set_lds_limit<Real, true, C, true>();
     }
     template<typename Real>
     void set_lds_limits()
@@ -1089,32 +1090,39 @@ class Batch
         set_lds_limits_class<Real, 0>();
         set_lds_limits_class<Real, 1>();
         set_lds_limits_class<Real, 2>();
+        if(sizeof(Real) == 8) {set_lds_limit<double, false, kRepWide, false>();}
     }
 
-    template<typename Real, bool ENERGY, int C>
-    void launch_shape(int nsteps, int eval_only)
+    template<typename Real, bool ENERGY, int C, bool TSP>
+    void launch_shape(size_t first, size_t count, int nsteps, int eval_only)
     {
-        constexpr int BS = Shape<Real, C>::bs, PPT = Shape<Real, C>::ppt;
-        static_assert(BS * PPT == (int)kRepClassMaxN[C], "class shape must cover its size");
-        // the class's replicas without 3SPN2 terms, then (same stream) those with them
+        using Shape = RepShape<Real, C, TSP>;
+        constexpr int cls = C == kRepWide ? 1 : C;
+        static_assert(Shape::bs * Shape::ppt == (int)kRepClassMaxN[cls], "class shape must cover its size");
+        if(count == 0) {return;}
+        hipLaunchKernelGGL((MJG_REP_KERNEL(Real, ENERGY, C, TSP)), dim3((uint32_t)count), dim3(Shape::bs), grp_lds_[cls],
+                           cls_stream_[cls], d_descs_ + first, nsteps, eval_only);
+    }
+    // the class's replicas without 3SPN2 terms, then (same stream) those with them
+    template<typename Real, bool ENERGY, int C>
+    void launch_shapes(int nsteps, int eval_only)
+    {
         const size_t plain = grp_count_[C] - grp_tsp_[C];
-        if(plain > 0)
+        // the middle FP64 class's two shapes: see RepShape
+        constexpr bool two_shapes = sizeof(Real) == 8 && !ENERGY && C == 1;
+        if(two_shapes && plain <= (size_t)n_cu_)
         {
-            hipLaunchKernelGGL((k_replica_segment<Real, ENERGY, BS, PPT, false>), dim3((uint32_t)plain), dim3(BS),
-                               grp_lds_[C], cls_stream_[C], d_descs_ + grp_first_[C], nsteps, eval_only);
+            launch_shape<Real, ENERGY, two_shapes ? kRepWide : C, false>(grp_first_[C], plain, nsteps, eval_only);
         }
-        if(grp_tsp_[C] > 0)
-        {
-            hipLaunchKernelGGL((k_replica_segment<Real, ENERGY, BS, PPT, true>), dim3((uint32_t)grp_tsp_[C]), dim3(BS),
-                               grp_lds_[C], cls_stream_[C], d_descs_ + grp_first_[C] + plain, nsteps, eval_only);
-        }
+        else {launch_shape<Real, ENERGY, C, false>(grp_first_[C], plain, nsteps, eval_only);}
+        launch_shape<Real, ENERGY, C, true>(grp_first_[C] + plain, grp_tsp_[C], nsteps, eval_only);
     }
     template<typename Real, bool ENERGY>
     void launch_class(int c, int nsteps, int eval_only)
     {
-        if(c == 0) {launch_shape<Real, ENERGY, 0>(nsteps, eval_only);}
-        else if(c == 1) {launch_shape<Real, ENERGY, 1>(nsteps, eval_only);}
-        else {launch_shape<Real, ENERGY, 2>(nsteps, eval_only);}
+        if(c == 0) {launch_shapes<Real, ENERGY, 0>(nsteps, eval_only);}
+        else if(c == 1) {launch_shapes<Real, ENERGY, 1>(nsteps, eval_only);}
+        else {launch_shapes<Real, ENERGY, 2>(nsteps, eval_only);}
     }
 
     // mode 0: step segment, 1: evaluate after a forced rebuild (set-up), 2: evaluate with energies.
@@ -1302,6 +1310,7 @@ class Batch
     hipStream_t stream_ = nullptr;                 // class 0's stream; set-up copies and joins
     hipStream_t cls_stream_[kRepClasses] = {};
     hipEvent_t ev_fork_ = nullptr, ev_join_[kRepClasses] = {};
+    int n_cu_ = 0;                                 // compute units of the device
     size_t grp_count_[kRepClasses] = {}, grp_first_[kRepClasses] = {}, grp_lds_[kRepClasses] = {};
     size_t grp_tsp_[kRepClasses] = {};             // replicas with 3SPN2 terms, last in their class
     std::vector<std::unique_ptr<Replica>> reps_;

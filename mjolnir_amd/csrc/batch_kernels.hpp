@@ -42,9 +42,9 @@ __host__ __device__ constexpr uint32_t grid_cells(uint32_t grid_bits) {return 1u
 constexpr uint32_t kRepClassMaxN[kRepClasses] = {256, 1024, 2048};
 
 // terms and list entries per thread per load round: one term and two list entries at 1024
-// threads (at most 128 VGPRs; larger batches spilled registers and measured 1-5 % slower) and at
-// 256 threads (no spill, three waves per SIMD; the same speed as four and eight); the FP64
-// kernel's 512-thread classes (256 VGPRs) take four and eight
+// threads (at most 128 VGPRs; larger batches measured up to 10 % slower) and at 256 threads (the
+// same speed as four and eight); the FP64 kernels' 512-thread classes (256 VGPRs) take four and
+// eight
 template<int BS> struct RepBatching
 {
     static constexpr int terms = (BS >= 1024 || BS == 256) ? 1 : 4;
@@ -1573,27 +1573,40 @@ k_replica_segment(const RepDesc* __restrict__ reps, int nsteps, int eval_only)
     else {rep_segment<Real, ENERGY, BS, PPT, TSP, false>(R, nsteps, eval_only, smem, sh);}
 }
 
-// Block shape of each size class: threads and particles per thread (the FP64 kernel needs more
-// registers per thread, so its two larger classes run 512 threads with 2 and 4 particles each).
-template<typename Real, int C> struct RepShape
+// Block shape of each size class: threads and particles per thread.  A replica is one workgroup,
+// bound by the latency of its phases, so the most threads that the registers allow are taken:
+// 1024, but 512 for the FP64 kernels with 3SPN2 terms (424-456 bytes of scratch at 1024 threads:
+// 400 replicas of 60 base pairs took 78.4 us a step at 512 threads and 87.5 at 1024).  The plain
+// FP64 kernel fits 124 registers at 1024 threads: 190 chains of up to 2000 particles 63.3 -> 52.1
+// us a step from 512 threads.  Its middle class fits both ways and is the exception: 700 chains
+// of up to 700 particles took 33.6 us at 512 threads and 38.3 at 1024, 256 of them 25.5 and
+// 21.7, so kRepWide is its 1024-thread shape, for launches of no more replicas than there are
+// CUs.  The shape changes no trajectory (integer force sums); the launches that evaluate
+// energies keep the class's own shape, so that the order of their sums depends on the replica alone.
+constexpr int kRepWide = 3;
+constexpr uint32_t rep_shape_n(int C) {return kRepClassMaxN[C == kRepWide ? 1 : C];}
+template<typename Real, int C, bool TSP> struct RepShape
 {
-    static constexpr int bs = C == 0 ? 256 : sizeof(Real) == 8 ? 512 : 1024;
-    static constexpr int ppt = (int)(kRepClassMaxN[C] / bs);
+    static constexpr int bs = C == 0 ? 256 : (sizeof(Real) == 8 && (TSP || C == 1)) ? 512 : 1024;
+    static constexpr int ppt = (int)(rep_shape_n(C) / bs);
 };
 
 // The kernel's instantiations: one per (Real, ENERGY, size class, TSP).  They are compiled in
 // separate translation units (batch_seg.hip, once per Real / ENERGY / TSP), and every other
 // translation unit only declares them.
 #define MJG_REP_KERNEL(Real, ENERGY, C, TSP) \
-    k_replica_segment<Real, ENERGY, RepShape<Real, C>::bs, RepShape<Real, C>::ppt, TSP>
+    k_replica_segment<Real, ENERGY, RepShape<Real, C, TSP>::bs, RepShape<Real, C, TSP>::ppt, TSP>
 #define MJG_REP_INSTANCES(PREFIX, Real, ENERGY, TSP) \
     PREFIX template __global__ void MJG_REP_KERNEL(Real, ENERGY, 0, TSP)(const RepDesc* __restrict__, int, int); \
     PREFIX template __global__ void MJG_REP_KERNEL(Real, ENERGY, 1, TSP)(const RepDesc* __restrict__, int, int); \
     PREFIX template __global__ void MJG_REP_KERNEL(Real, ENERGY, 2, TSP)(const RepDesc* __restrict__, int, int);
+#define MJG_REP_WIDE_INSTANCE(PREFIX) \
+    PREFIX template __global__ void MJG_REP_KERNEL(double, false, kRepWide, false)(const RepDesc* __restrict__, int, int);
 #define MJG_REP_ALL_INSTANCES(PREFIX) \
     MJG_REP_INSTANCES(PREFIX, float, false, false) MJG_REP_INSTANCES(PREFIX, float, false, true) \
     MJG_REP_INSTANCES(PREFIX, float, true, false) MJG_REP_INSTANCES(PREFIX, float, true, true) \
     MJG_REP_INSTANCES(PREFIX, double, false, false) MJG_REP_INSTANCES(PREFIX, double, false, true) \
-    MJG_REP_INSTANCES(PREFIX, double, true, false) MJG_REP_INSTANCES(PREFIX, double, true, true)
+    MJG_REP_INSTANCES(PREFIX, double, true, false) MJG_REP_INSTANCES(PREFIX, double, true, true) \
+    MJG_REP_WIDE_INSTANCE(PREFIX)
 
 } // mjg

@@ -121,3 +121,28 @@ def test_exclusions_far_apart_in_index():
                       attributes={"temperature": 300.0}, local=[hub], global_=[ev],
                       integrator=IntegratorSpec("BAOABLangevin", 0.01, np.full(n, 0.1), seed=2), name="hub")
     _follow(spec, 120)
+
+
+def test_replica_block_shapes_agree():
+    """FP64 replicas of 257 to 1024 particles run 1024 threads while there are no more of them than CUs
+    (256), else 512; larger ones 1024.  Forces are integer sums, so a trajectory is the same bit for bit
+    in both shapes, and it follows the oracle's."""
+    import oracle
+    from mjolnir_amd import capi, workloads
+    targets = [workloads.cg_chain(n, seed=n, max_bend_deg=150.0) for n in (257, 700, 1024, 1025, 2048)]
+    filler = [workloads.cg_chain(258, seed=1, max_bend_deg=150.0)] * 254      # 257 replicas of the middle class
+    out = []
+    for specs in (targets, targets + filler):
+        b = capi.Batch(capi.FP64)
+        ids = [b.add(s) for s in specs][:len(targets)]
+        b.initialize()
+        b.step(60)
+        out.append([b.state(r) for r in ids])
+        b.close()
+    for spec, few, many in zip(targets, *out):
+        assert all(np.array_equal(a, c) for a, c in zip(few, many)), spec.name
+        o = oracle.OracleEngine(spec)
+        o.step(60)
+        xo, vo, fo = o.state()
+        # as the other FP64 replica trajectories (fixed-point sums in units of 2^-32)
+        assert np.abs(few[0] - xo).max() < 1e-7 and np.abs(few[1] - vo).max() < 1e-7, spec.name
