@@ -292,14 +292,7 @@ struct PairParams
     int npar;                // per-particle parameter columns
 };
 
-// Per-particle pair parameters of a pair term, read through an accessor: column c of the
-// parameter row `key`.  GlobalPar reads the engine's per-particle table (key = particle index);
-// the cell-tile kernel reads the copies it staged in LDS (key = staging slot).
-template<int NPAR> struct GlobalPar
-{
-    const double* __restrict__ p;
-    __device__ __forceinline__ double get(uint32_t key, int c) const {return p[(size_t)NPAR * key + c];}
-};
+// Per-particle pair parameters of a pair term: column c of the parameter row `key`.
 template<int KIND> constexpr int pair_npar() {return KIND == kPairLJ ? 2 : 1;}
 // the parameters of one pair in registers: key 0 the owner, key 1 the partner
 struct RegPar
@@ -401,7 +394,7 @@ __device__ __forceinline__ void pair_term_p(const PairParams& pp, uint32_t i, ui
 // interaction; inside a segment `tpp` lanes share one participant (sorted slot t), split its
 // row nl[t * cap + k] with stride tpp, and combine their partial forces with a fixed
 // butterfly, so the sum order is fixed.  The interaction's force on i lands in its own array
-// fout[i] (zero for non-participants), which k_finish adds up.
+// fout[i] (zero for non-participants), which the gather of k_advance or k_finish adds up.
 // ------------------------------------------------------------------------------------
 struct PairSeg
 {

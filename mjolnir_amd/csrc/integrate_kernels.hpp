@@ -2,11 +2,9 @@
 //
 // k_baoab_a / k_gjf_a are the per-particle loops before the force call
 // (BAOABLangevinIntegrator.hpp:176-200, GJFNVTLangevinIntegrator.hpp:172-197) fused with the
-// largest-displacement reduction; k_margin is ForceField::reduce_margin on every partition
-// (ForceField.hpp:75-92, PeriodicGridCellList.hpp:100-110) decided on the device, so a step
-// never waits for the host; k_kick_b / k_gjf_b are the velocity updates after the force call
-// (BAOABLangevinIntegrator.hpp:222-229, GJFNVTLangevinIntegrator.hpp:222-229); k_ul_a /
-// k_ul_accel are UnderdampedLangevin's two per-particle loops.  The noise is the engine's
+// largest-displacement reduction, for steps that a motion remover ends; steps without one are
+// joined by k_advance (step_kernels.hpp).  k_ul_a / k_ul_accel are UnderdampedLangevin's two
+// per-particle loops.  The noise is the engine's
 // Philox stream indexed by (seed, step, particle).
 #pragma once
 #include "device_common.hpp"
@@ -178,7 +176,7 @@ k_ul_accel(uint32_t n, double4* __restrict__ vel, double4* __restrict__ accel, c
 }
 
 // The velocity half-kick after the force call is part of k_finish (force_kernels.hpp), and
-// the skin check is part of k_prep_small / k_margin_large (nlist_kernels.hpp).
+// the skin check is part of k_prep_small / k_margin_large (nlist_kernels.hpp) and k_forces.
 
 __global__ void __launch_bounds__(256)
 k_kinetic(uint32_t n, const double4* __restrict__ vel, const double* __restrict__ mass, double* __restrict__ out)

@@ -1,7 +1,7 @@
 // Cell-tile pair kernel of the engine (periodic cell lists).
 //
-// One workgroup per cell of the interaction's grid.  It stages the positions, per-particle
-// parameters and particle indices of the 27 surrounding cells in LDS, in the order the list
+// One workgroup per cell of the interaction's grid.  It stages the 27 surrounding cells' slots
+// (TileSlot, written in slot order by k_tile_slots each step) in LDS, in the order the list
 // build walks them (z outer, then y, then x; each cell's sorted slots in order), and walks the
 // rows of its own cell's participants.  A row entry's staging slot is written by k_verlet beside
 // its particle index (nl16), so a partner is read from LDS instead of gathered from global memory:
