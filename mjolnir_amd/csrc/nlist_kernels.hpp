@@ -708,8 +708,10 @@ k_prep_small(const double4* __restrict__ pos, PrepSegTable tab, StepCtl* __restr
             }
             double w = s.r_list * (1.0 + 1e-6);
             if(!(w > 0.0)) {w = 1.0;}
+            // widened until the grid fits the LDS tables, however far apart the participants are (an
+            // exploded chain spans 1e11 A): ext is finite, so w outgrows it and the loop ends
             int dim[3];
-            for(int it = 0; it < 200; ++it)
+            for(;;)
             {
                 unsigned long long prod = 1;
                 for(int d = 0; d < 3; ++d)

@@ -146,3 +146,30 @@ def test_replica_block_shapes_agree():
         xo, vo, fo = o.state()
         # as the other FP64 replica trajectories (fixed-point sums in units of 2^-32)
         assert np.abs(few[0] - xo).max() < 1e-7 and np.abs(few[1] - vo).max() < 1e-7, spec.name
+
+
+def test_cell_grid_of_participants_far_apart():
+    """An open box whose participants span 1e13 A in every direction (an exploded chain reaches 1e10): the
+    one-workgroup rebuild widens its cells until they fit its tables, and the list is the all-pairs list.
+    The list's cells would have to be 1e8 times the list radius wide to fit after a bounded widening."""
+    from mjolnir_amd import capi
+    from mjolnir_amd.spec import GlobalSpec, IntegratorSpec, SystemSpec
+    rng = np.random.default_rng(7)
+    g = np.stack(np.meshgrid(*[np.arange(2)] * 3, indexing="ij"), -1).reshape(-1, 3) * 1.1
+    far = np.concatenate([np.zeros((1, 3)), rng.uniform(-1e13, 1e13, size=(20, 3))])
+    pos = np.concatenate([g + c for c in far])
+    n = len(pos)
+
+    def engine(partition):
+        lj = GlobalSpec(potential="LennardJones", participants=np.arange(n), params=np.tile([1.0, 0.02], (n, 1)),
+                        cutoff=2.5, partition=partition, margin=0.5)
+        return capi.Engine(SystemSpec(boundary="unlimited", mass=np.ones(n), pos=pos, vel=np.zeros_like(pos),
+                                      attributes={"temperature": 1.0}, global_=[lj],
+                                      integrator=IntegratorSpec("BAOABLangevin", 0.01, np.full(n, 0.01), seed=3),
+                                      name=f"far_{partition}"))
+
+    cells, plain = engine("CellList"), engine("VerletList")
+    assert len(cells.pairs(0)) >= 28 and np.array_equal(cells.pairs(0), plain.pairs(0))
+    fc, fp = cells.state()[2], plain.state()[2]
+    # the same pairs in another order: rounding of sums of up to 7 partners
+    assert np.abs(fc - fp).max() <= 1e-14 * np.abs(fp).max()
