@@ -471,7 +471,8 @@ void Engine::alloc_list(GlobalIA& g, uint32_t cap)
 // The cell-tile pair kernel (tile_kernels.hpp) serves a pair interaction on a periodic cell list
 // with at least kTileMinNp participants (MJG_TILE_MIN_NP overrides it; MJG_NO_TILE=1 turns the
 // kernel off): it needs a launch of one workgroup per cell, which fills the GPU only for large
-// grids.  Its staging capacity starts at twice the mean 27-cell neighbourhood and grows with the
+// grids.  In the mixed precision no axis of the box may be narrower than three list radii
+// (GlobalIA::one_image): the gather kernel serves those boxes.  Its staging capacity starts at twice the mean 27-cell neighbourhood and grows with the
 // largest one a build reports (ListCtl::maxnbr), up to what the LDS of one workgroup holds after
 // the kernel's static LDS (224 bytes in the current build; 4 KiB are set aside for it).
 constexpr uint32_t kTileMinNp = 16384;
@@ -624,12 +625,18 @@ void Engine::setup_global(GlobalIA& g)
               !(no_tile && no_tile[0] == '1');
     if(g.tiled)
     {
-        const double mean_nbr = 27.0 * (double)np / (double)g.grid.ncell;
-        g.fast_build = true;
+        g.one_image = true;
         for(int d = 0; d < 3; ++d)
         {
-            g.fast_build = g.fast_build && (g.grid.dim[d] - 2) * (box_.width[d] / g.grid.dim[d]) >= g.r_list;
+            g.one_image = g.one_image && (g.grid.dim[d] - 2) * (box_.width[d] / g.grid.dim[d]) >= g.r_list;
         }
+        // the mixed kernel takes each neighbour cell at one image and needs that to be the nearest; the
+        // FP64 kernel forms the minimum image of every pair
+        g.tiled = g.one_image || precision_ != MJG_FP32_FIXED;
+    }
+    if(g.tiled)
+    {
+        const double mean_nbr = 27.0 * (double)np / (double)g.grid.ncell;
         g.tile_cap = (uint32_t)std::min<double>(kTileMaxCap, std::max(256.0, 1.25 * mean_nbr + 64.0));
         // MJG_TILE_CAP fixes the staging capacity (no growth): a capacity below the largest
         // neighbourhood serves every build from global memory
@@ -825,7 +832,7 @@ void Engine::launch_rebuilds(int force, uint32_t k)
         if(!g.tiled) {continue;}
         const ListSeg s = list_seg(g, gi);
         const uint32_t blocks = std::min<uint32_t>(blocks_for(g.grid.ncell, kXcds) * kXcds, kVerletMaxBlocks);
-        if(g.fast_build)
+        if(g.one_image)
         {
             hipLaunchKernelGGL(k_verlet_tiled<true>, dim3(blocks), dim3(kTileThreads),
                                (size_t)g.tile_cap * kBuildBytesPerParticleF32, stream_, d_pos_, box_, s, g.tile_cap);

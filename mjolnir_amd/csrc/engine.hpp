@@ -83,7 +83,9 @@ struct GlobalIA
     void* d_slots = nullptr;  // positions and parameters in slot order (k_tile_slots)
     uint32_t tile_cap = 0;
     bool tile_fixed = false;
-    bool fast_build = false;      // the grid allows the FP32 tests of k_verlet_tiled
+    // no pair within r_list is nearer through another image of its neighbour cell: (dim - 2) cell widths
+    // are at least r_list on every axis.  The mixed kernel and the FP32 tests of k_verlet_tiled need it.
+    bool one_image = false;
     bool multibody() const {return pot == kBasePair || pot == kCrossStack;}
 };
 

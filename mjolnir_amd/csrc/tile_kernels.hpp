@@ -404,7 +404,11 @@ k_tile_slots(const double4* __restrict__ pos, Box box, const uint32_t* __restric
         // A particle has moved less than half the skin since the build that put it in this cell, and
         // positions are wrapped into the box every step: its image nearest to the cell's centre is the one
         // within half a cell plus that drift, fewer than half a box width, since a periodic grid has at
-        // least three cells a dimension.
+        // least three cells a dimension.  Seen from a neighbouring home cell this image is a partner's nearest
+        // one, or out of reach, where (dim - 2) cell widths are at least r_list on every axis: the other
+        // image lies (dim - 2) widths away at the build and r_list less the skin, the cutoff, later.  An
+        // axis of three cells narrower than r_list has pairs inside the cutoff through its other side;
+        // this kernel is not launched for such boxes.
         const Grid g = *grid;
         const uint32_t cell = skeys[t];
         const int cx = (int)(cell % (uint32_t)g.dim[0]);

@@ -173,3 +173,52 @@ def test_cell_grid_of_participants_far_apart():
     fc, fp = cells.state()[2], plain.state()[2]
     # the same pairs in another order: rounding of sums of up to 7 partners
     assert np.abs(fc - fp).max() <= 1e-14 * np.abs(fp).max()
+
+
+def _fluid(potential, n, margin, seed, box=None):
+    """n particles of one pair potential on a jittered lattice in a periodic box (cubic unless given)."""
+    from mjolnir_amd import workloads
+    from mjolnir_amd.spec import GlobalSpec, IntegratorSpec, SystemSpec
+    rng = np.random.default_rng(seed)
+    spacing = {"LennardJones": 4.74, "ExcludedVolume": 5.0, "DebyeHuckel": 6.0, "3SPN2ExcludedVolume": 5.5}[potential]
+    if box is None:
+        side = int(np.ceil(n ** (1 / 3) - 1e-9))
+        sites = (side, side, side)
+    else:
+        sites = tuple(int(w / spacing) for w in box)
+    g = np.stack(np.meshgrid(*[np.arange(k) for k in sites], indexing="ij"), -1).reshape(-1, 3)[:n]
+    upper = np.array(box if box is not None else [s * spacing for s in sites], dtype=float)
+    pos = (g + 0.5) * (upper / np.array(sites)) + rng.uniform(-0.3, 0.3, size=g.shape)
+    n = len(pos)
+    par, kw = {"LennardJones": (np.tile([4.0, 0.2], (n, 1)), {}),
+               "ExcludedVolume": (rng.uniform(1.6, 2.0, size=(n, 1)), {"epsilon": 0.2}),
+               "DebyeHuckel": (rng.choice([-1.0, 1.0], size=(n, 1)), {"cutoff": 2.0}),
+               "3SPN2ExcludedVolume": (rng.integers(0, 6, size=(n, 1)).astype(float), {})}[potential]
+    pair = GlobalSpec(potential=potential, participants=np.arange(n), params=par, partition="CellList", margin=margin, **kw)
+    mass = np.ones(n)
+    return SystemSpec(boundary="periodic", mass=mass, pos=pos, vel=workloads.maxwell_boltzmann(rng, mass, 300.0),
+                      lower=np.zeros(3), upper=upper, attributes={"temperature": 300.0, "ionic_strength": 0.5},
+                      global_=[pair], integrator=IntegratorSpec("BAOABLangevin", 0.01, np.full(n, 0.1), seed=seed),
+                      name=f"{potential}_{n}")
+
+
+THIN = (62.0, 60.0, 27.0)      # r_list = 15: the third axis' three cells are 9 A wide
+
+
+def test_mixed_forces_in_a_box_narrower_than_three_list_radii(monkeypatch):
+    """An axis clamped to three cells: a pair of neighbouring cells can be nearer through the other side of the
+    box, which the mixed cell-tile kernel's staging (one image a cell) would miss.  Bar: the mixed path's
+    1e-5 of the RMS force."""
+    from mjolnir_amd import capi
+    monkeypatch.setenv("MJG_TILE_MIN_NP", "0")
+    spec = _fluid("LennardJones", 10 ** 6, 0.5, 3, THIN)
+    e = capi.Engine(spec, capi.FP32_FIXED)
+    for steps in (0, 40):
+        e.step(steps)
+        x, _, f = e.state()
+        ref = capi.Engine(dataclasses.replace(spec, pos=x), capi.FP64, with_integrator=False)
+        ref.calc_force()
+        want = ref.state()[2]
+        rms = float(np.sqrt(np.mean((f - want) ** 2) / np.mean(want ** 2)))
+        print(f"[gpu] thin box N={spec.n} after {steps} steps: mixed RMS error {rms:.1e}", flush=True)
+        assert rms < 1e-5
