@@ -48,7 +48,8 @@ __device__ __forceinline__ double from_ordered_bits(unsigned long long b)
 struct ListCtl
 {
     int rebuild;                   // 1: rebuild this step
-    unsigned int maxcount;         // largest partner count seen at the last build
+    unsigned int maxcount;         // largest partner count of any build since the last forced one: the host
+                                   // looks once a segment, and a row cut short by any of its builds counts
     unsigned int maxnbr;           // largest 27-cell neighbourhood of a row at the last build
     unsigned long long bbox_min[3];
     unsigned long long bbox_max[3];
@@ -643,7 +644,7 @@ __device__ __forceinline__ int margin_decision(ListCtl& c, double dmargin, doubl
     const double m = c.margin - dmargin;
     if(m < 0)
     {
-        c.rebuild = 1; c.margin = abs_margin; c.maxcount = 0; c.maxnbr = 0;
+        c.rebuild = 1; c.margin = abs_margin; c.maxnbr = 0;
         for(int d = 0; d < 3; ++d) {c.bbox_min[d] = ~0ull; c.bbox_max[d] = 0ull;}
         return 1;
     }

@@ -222,3 +222,53 @@ def test_mixed_forces_in_a_box_narrower_than_three_list_radii(monkeypatch):
         rms = float(np.sqrt(np.mean((f - want) ** 2) / np.mean(want ** 2)))
         print(f"[gpu] thin box N={spec.n} after {steps} steps: mixed RMS error {rms:.1e}", flush=True)
         assert rms < 1e-5
+
+
+def _crossing_clusters(boundary, filler, remove=False):
+    """Two clusters of 48 that fly through each other within 100 steps: the rows hold 47 partners before and
+    after and up to 95 in between, above the first row length of 64.  The filler (a lattice of single
+    particles beyond each other's list radius) only makes the interaction large."""
+    from mjolnir_amd.spec import GlobalSpec, IntegratorSpec, SystemSpec
+    g = np.stack(np.meshgrid(np.arange(4), np.arange(4), np.arange(3), indexing="ij"), -1).reshape(-1, 3) * 1.3
+    centre = np.array([48.0, 48.0, 121.0])
+    pos = np.concatenate([g - [6.0, 0, 0], g + [6.0, 0.6, 0.6]]) + centre
+    vel = np.zeros_like(pos)
+    vel[:48, 0], vel[48:, 0] = 12.0, -12.0
+    if filler:
+        f = np.stack(np.meshgrid(np.arange(16), np.arange(16), np.arange(17), indexing="ij"), -1).reshape(-1, 3)[:filler]
+        pos = np.concatenate([pos, (f + 0.5) * 6.0])
+        vel = np.concatenate([vel, np.zeros((filler, 3))])
+    n = len(pos)
+    lj = GlobalSpec(potential="LennardJones", participants=np.arange(n), params=np.tile([1.0, 0.02], (n, 1)), cutoff=2.5,
+                    partition="CellList", margin=1.0)
+    return SystemSpec(boundary=boundary, mass=np.ones(n), pos=pos, vel=vel, lower=np.zeros(3),
+                      upper=np.array([96.0, 96.0, 140.0]), attributes={"temperature": 1.0}, global_=[lj],
+                      integrator=IntegratorSpec("BAOABLangevin", 0.01, np.full(n, 0.01), seed=3,
+                                                remove=(remove, False, False)), name=f"crossing_{boundary}_{n}")
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("case", ["open", "periodic", "tile", "small_separate"])
+def test_rows_outgrown_by_a_build_between_two_that_fit(case, precision, monkeypatch):
+    """Every build of a segment counts, not only its last: the segment runs again with longer rows.  The tile
+    case fixes a staging capacity that the neighbourhoods exceed in the middle of the segment as well, so that
+    its rows are served from global memory and from the staged tile in turn."""
+    import oracle
+    from mjolnir_amd import capi
+    if case == "tile":
+        monkeypatch.setenv("MJG_TILE_MIN_NP", "0")
+        monkeypatch.setenv("MJG_TILE_CAP", "70")
+    spec = _crossing_clusters("periodic" if case in ("periodic", "tile") else "unlimited",
+                              0 if case == "small_separate" else 4200, remove=case == "small_separate")
+    e, o = capi.Engine(spec, capi.FP64 if precision == "fp64" else capi.FP32_FIXED), oracle.OracleEngine(spec)
+    built = e.counters()[1]
+    e.step(100)
+    o.step(100)
+    (x, v, _), (xo, vo, _) = e.state(), o.state()
+    dx, dv = float(np.abs(x - xo).max()), float(np.abs(v - vo).max())
+    print(f"[gpu] {spec.name} {case} {precision}: dx {dx:.1e} dv {dv:.1e} rebuilds {e.counters()[1] - built}", flush=True)
+    # FP64: rounding; mixed: forces of up to about 10 kcal/mol/A at 1e-6 of themselves over one time unit
+    tol = 1e-8 if precision == "fp64" else 1e-4
+    assert dx < tol and dv < tol
+    assert np.abs(vo[:48, 0] - 12.0).max() > 0.05              # the clusters did feel each other
+    assert e.counters()[1] - built >= 5
