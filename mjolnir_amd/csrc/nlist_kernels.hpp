@@ -636,15 +636,13 @@ struct PrepSegTable
 __device__ __forceinline__ int margin_decision(ListCtl& c, double dmargin, double abs_margin, int never, int force)
 {
     if(never && !force) {c.rebuild = 0; return 0;}
-    if(force)
-    {
-        c.rebuild = 1; c.margin = never ? INFINITY : abs_margin; c.maxcount = 0; c.maxnbr = 0;
-        return 1;
-    }
     const double m = c.margin - dmargin;
-    if(m < 0)
+    if(force || m < 0)
     {
-        c.rebuild = 1; c.margin = abs_margin; c.maxnbr = 0;
+        c.rebuild = 1;
+        c.margin = never ? INFINITY : abs_margin;
+        if(force) {c.maxcount = 0;}
+        c.maxnbr = 0;
         for(int d = 0; d < 3; ++d) {c.bbox_min[d] = ~0ull; c.bbox_max[d] = 0ull;}
         return 1;
     }

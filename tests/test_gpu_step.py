@@ -272,3 +272,23 @@ def test_rows_outgrown_by_a_build_between_two_that_fit(case, precision, monkeypa
     assert dx < tol and dv < tol
     assert np.abs(vo[:48, 0] - 12.0).max() > 0.05              # the clusters did feel each other
     assert e.counters()[1] - built >= 5
+
+
+def test_open_system_above_the_one_workgroup_rebuild_is_set_up_through_its_grid():
+    """The first build of a large open system finds its own bounding box.  With all 50,000 participants in one
+    cell the set-up took 100 s, most of it one lane's sort; through the grid it takes a few milliseconds."""
+    import time
+    from mjolnir_amd import capi
+    spec = _crossing_clusters("unlimited", 4200)
+    f = np.stack(np.meshgrid(*[np.arange(36)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    pos = np.concatenate([spec.pos, (f + 0.5) * 6.0 + [0.0, 0.0, 200.0]])
+    n = len(pos)
+    g = dataclasses.replace(spec.global_[0], participants=np.arange(n), params=np.tile([1.0, 0.02], (n, 1)))
+    spec = dataclasses.replace(spec, pos=pos, vel=np.zeros_like(pos), mass=np.ones(n), global_=[g],
+                               integrator=dataclasses.replace(spec.integrator, coefs=np.full(n, 0.01)))
+    t0 = time.perf_counter()
+    e = capi.Engine(spec)
+    took = time.perf_counter() - t0
+    print(f"[gpu] open system of {n}: set up in {took:.2f} s", flush=True)
+    assert took < 10.0
+    assert len(e.pairs(0)) > 48 * 40 and e.pairs(0).max() < 96       # the clusters' pairs alone
