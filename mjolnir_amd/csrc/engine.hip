@@ -663,10 +663,11 @@ void Engine::setup_global(GlobalIA& g)
     if(g.multibody()) {g.d_acc = dalloc<unsigned long long>(3 * n_ + 1);}   // sums and the flag word
     sync();
     g.tpp = 8;
-    // the first row length: a quarter above the mean of a periodic cell list (a liquid's longest row), so
-    // that its first build is kept; grown where a row is longer
+    // the first row length: 1.3 times the mean of a periodic cell list and 24 (a liquid's longest row), so
+    // that its first build is kept; grown where a row is longer.  Not where a rule on molecules or bases
+    // drops most partners: memory for them all could be more than there is.
     uint32_t cap = 64;
-    if(box_.periodic && g.partition == MJG_PART_CELLLIST)
+    if(box_.periodic && g.partition == MJG_PART_CELLLIST && g.rule.ignore_mol == 0 && g.rule.base_rule != 2)
     {
         const double volume = box_.width[0] * box_.width[1] * box_.width[2];
         const double mean = (double)np * (4.0 / 3.0 * 3.14159265358979323846) * g.r_list * g.r_list * g.r_list / volume;

@@ -274,21 +274,49 @@ def test_rows_outgrown_by_a_build_between_two_that_fit(case, precision, monkeypa
     assert e.counters()[1] - built >= 5
 
 
+def _open_crossing_among(extra):
+    """The crossing clusters in an open box among 4200 + extra^3 single particles."""
+    spec = _crossing_clusters("unlimited", 4200)
+    f = np.stack(np.meshgrid(*[np.arange(extra)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    more = (f + 0.5) * 6.0 + [0.0, 0.0, 200.0]
+    n = spec.n + len(more)
+    g = dataclasses.replace(spec.global_[0], participants=np.arange(n), params=np.tile([1.0, 0.02], (n, 1)))
+    return dataclasses.replace(spec, pos=np.concatenate([spec.pos, more]), vel=np.concatenate([spec.vel, np.zeros_like(more)]),
+                               mass=np.ones(n), global_=[g],
+                               integrator=dataclasses.replace(spec.integrator, coefs=np.full(n, 0.01)))
+
+
 def test_open_system_above_the_one_workgroup_rebuild_is_set_up_through_its_grid():
     """The first build of a large open system finds its own bounding box.  With all 50,000 participants in one
     cell the set-up took 100 s, most of it one lane's sort; through the grid it takes a few milliseconds."""
     import time
     from mjolnir_amd import capi
-    spec = _crossing_clusters("unlimited", 4200)
-    f = np.stack(np.meshgrid(*[np.arange(36)] * 3, indexing="ij"), -1).reshape(-1, 3)
-    pos = np.concatenate([spec.pos, (f + 0.5) * 6.0 + [0.0, 0.0, 200.0]])
-    n = len(pos)
-    g = dataclasses.replace(spec.global_[0], participants=np.arange(n), params=np.tile([1.0, 0.02], (n, 1)))
-    spec = dataclasses.replace(spec, pos=pos, vel=np.zeros_like(pos), mass=np.ones(n), global_=[g],
-                               integrator=dataclasses.replace(spec.integrator, coefs=np.full(n, 0.01)))
+    spec = _open_crossing_among(36)
     t0 = time.perf_counter()
     e = capi.Engine(spec)
     took = time.perf_counter() - t0
-    print(f"[gpu] open system of {n}: set up in {took:.2f} s", flush=True)
+    print(f"[gpu] open system of {spec.n}: set up in {took:.2f} s", flush=True)
     assert took < 10.0
     assert len(e.pairs(0)) > 48 * 40 and e.pairs(0).max() < 96       # the clusters' pairs alone
+
+
+def _used():
+    """Bytes of the device in use, asked of the HIP runtime that the library has loaded."""
+    import ctypes
+    from mjolnir_amd import capi
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert capi.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return total.value - free.value
+
+
+def test_first_rows_of_a_list_that_drops_other_molecules():
+    """Most partners within a large list radius belong to other molecules, which the interaction ignores (here
+    all of them: rows of 19,000 words would be 1.5 GB, and as much again beside them)."""
+    from mjolnir_amd import capi, workloads
+    spec = workloads.lj_fluid(n=20000, seed=2, cutoff=12.0)
+    spec.global_[0].ignore_molecule = "Others"
+    before = _used()
+    e = capi.Engine(spec)
+    used = _used() - before
+    print(f"[gpu] engine of {spec.n} particles: {used / 2 ** 20:.1f} MB", flush=True)
+    assert used < 3e8 and len(e.pairs(0)) == 0
