@@ -64,13 +64,22 @@ template<typename T> T* Engine::dalloc(size_t n)
         (void)hipGetLastError();
         throw std::bad_alloc();
     }
-    allocations_.push_back(p);
+    (share ? chunks_ : allocations_).push_back(p);
     if(share)
     {
         chunk_ = static_cast<char*>(p) + bytes;
         chunk_left_ = kChunk - bytes;
     }
     return static_cast<T*>(p);
+}
+// An array that is no longer used: an allocation of its own goes back to the device, a part of a shared
+// chunk stays with the engine.  Nothing may be running that reads it.
+void Engine::drelease(void* p)
+{
+    const auto at = std::find(allocations_.begin(), allocations_.end(), p);
+    if(p == nullptr || at == allocations_.end()) {return;}
+    (void)hipFree(p);
+    allocations_.erase(at);
 }
 // pinned host memory that kernels write small results to
 template<typename T> T* Engine::halloc(size_t n)
@@ -150,6 +159,7 @@ Engine::~Engine()
     if(graph_exec_) {(void)hipGraphExecDestroy(graph_exec_);}
     if(stream_) {(void)hipStreamSynchronize(stream_);}
     for(void* p : allocations_) {(void)hipFree(p);}
+    for(void* p : chunks_) {(void)hipFree(p);}
     for(void* p : host_allocations_) {(void)hipHostFree(p);}
     if(stream_) {(void)hipStreamDestroy(stream_);}
 }
@@ -456,16 +466,19 @@ void Engine::make_exclusions(GlobalIA& g)
     upload(g.d_mol, mol_.data(), n_);
 }
 
+// Rows of `cap` words.  The new arrays come first: where they are not to be had the list keeps its old
+// ones and their length.  A captured step holds the old ones and goes with them.
 void Engine::alloc_list(GlobalIA& g, uint32_t cap)
 {
-    const uint32_t np = (uint32_t)g.part.size();
+    const size_t words = g.part.size() * (size_t)cap;
+    uint32_t* nl = dalloc<uint32_t>(words);
+    uint16_t* nl16 = g.tiled ? dalloc<uint16_t>(words) : nullptr;
+    uint32_t* in = (g.inner && !g.tiled) ? dalloc<uint32_t>(words) : nullptr;
+    uint16_t* in16 = (g.inner && g.tiled) ? dalloc<uint16_t>(words) : nullptr;
+    if(graph_exec_) {(void)hipGraphExecDestroy(graph_exec_); graph_exec_ = nullptr;}
+    for(void* old : {(void*)g.d_nl, (void*)g.d_nl16, (void*)g.d_in, (void*)g.d_in16}) {drelease(old);}
     g.cap = cap;
-    g.d_nl = dalloc<uint32_t>((size_t)np * cap);
-    if(g.tiled) {g.d_nl16 = dalloc<uint16_t>((size_t)np * cap);}
-    if(g.inner)
-    {
-        if(g.tiled) {g.d_in16 = dalloc<uint16_t>((size_t)np * cap);} else {g.d_in = dalloc<uint32_t>((size_t)np * cap);}
-    }
+    g.d_nl = nl; g.d_nl16 = nl16; g.d_in = in; g.d_in16 = in16;
 }
 
 // The cell-tile pair kernel (tile_kernels.hpp) serves a pair interaction on a periodic cell list

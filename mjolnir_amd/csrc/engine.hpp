@@ -175,6 +175,7 @@ class Engine
     void sync();
     void check(hipError_t e, const char* what);
     template<typename T> T* dalloc(size_t n);
+    void drelease(void* p);
     template<typename T> T* halloc(size_t n);
     template<typename T> void upload(T* d, const T* h, size_t n);
     template<typename T> void download(T* h, const T* d, size_t n);
@@ -186,7 +187,7 @@ class Engine
     StateTransfer transfer_;
     double* h_energy_ = nullptr;   // pinned: per interaction, then the kinetic energy
     int* h_flag_ = nullptr;        // pinned: a kernel's decision for the host
-    std::vector<void*> allocations_, host_allocations_;
+    std::vector<void*> allocations_, chunks_, host_allocations_;
     static constexpr size_t kChunk = size_t(1) << 18;   // shared chunk of small device arrays
     char* chunk_ = nullptr;                              // its unused rest
     size_t chunk_left_ = 0;

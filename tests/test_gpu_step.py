@@ -309,6 +309,22 @@ def _used():
     return total.value - free.value
 
 
+def test_grown_rows_give_the_old_ones_back():
+    """The crossing clusters among 50,000 single particles: growing the rows (64 words, then about 130, in the
+    list and in the inner list) costs the difference, within 8 MB; the old rows are 26 MB."""
+    from mjolnir_amd import capi
+    spec = _open_crossing_among(36)
+    n = spec.n
+    e = capi.Engine(spec)
+    e.step(20)
+    before = _used()
+    e.step(80)
+    grown = _used() - before
+    rows = 95 + 95 // 4 + 16
+    print(f"[gpu] {n} particles: {grown / 2 ** 20:.1f} MB more after growing", flush=True)
+    assert grown < 2 * n * 4 * (rows - 64) + 8e6
+
+
 def test_first_rows_of_a_list_that_drops_other_molecules():
     """Most partners within a large list radius belong to other molecules, which the interaction ignores (here
     all of them: rows of 19,000 words would be 1.5 GB, and as much again beside them)."""
