@@ -511,6 +511,21 @@ static uint32_t lanes_for(uint32_t maxcount)
     return t;
 }
 
+// Lanes per row where k_forces keeps the list: as many as the row's partners ask for, and enough for its
+// rebuilds, in which the row's lanes share all np candidates.  Short rows have few lanes otherwise, and
+// few lanes rebuild slowly and leave the chip idle (4096 particles with one lane a row: 16 workgroups,
+// 1.3 ms).  Rebuilds come the more often the smaller the margin, so up to m = 0.1 a lane takes at most 128
+// candidates, at the usual 0.5 640.  Measured per FP64 step with the partners' lanes alone, and with these:
+// a fluid of 4096 at m = 0.05 34.6 -> 16.0 us, one of a twelfth of its density 175 -> 15.2 (the separate
+// rebuild kernels took 26.0 and 26.8); a chain of 4000 beads at m = 0.02 86 -> 24; a 650-bp duplex 138 -> 27,
+// at m = 0.5 18.1 -> 18.3 (20.4 with 128 candidates at every margin).
+static uint32_t self_lanes(uint32_t np, uint32_t lanes, double margin)
+{
+    const double tests = 128 * std::max(1.0, 10 * margin);
+    while(lanes < 64 && lanes * tests < np) {lanes <<= 1;}
+    return lanes;
+}
+
 void Engine::setup_global(GlobalIA& g)
 {
     const uint32_t np = (uint32_t)g.part.size();
@@ -1562,7 +1577,8 @@ void Engine::launch_step_forces(uint32_t k)
             RowSeg& r = a.row[a.nrow++];
             r.block_begin = block;
             r.never = (g.partition == MJG_PART_NAIVE);
-            r.p.kind = g.pot; r.p.tpp = g.multibody() ? g.mb_tpp : g.tpp; r.p.np = (uint32_t)g.part.size(); r.p.cap = g.cap;
+            r.p.kind = g.pot; r.p.np = (uint32_t)g.part.size(); r.p.cap = g.cap;
+            r.p.tpp = g.multibody() ? g.mb_tpp : self_lanes(r.p.np, g.tpp, g.margin);
             r.p.spart = g.d_spart; r.p.nl = g.d_nl; r.p.nn = g.d_nn; r.p.ppar = g.d_ppar; r.p.fout = g.d_fg;
             r.p.pp = g.pp;
             r.acc = g.d_acc;
