@@ -169,27 +169,20 @@ void Engine::set_state(const double* mass, const double* pos, const double* vel)
     if(!mass || !pos || !vel) {throw std::invalid_argument("null state pointer");}
     mass_.assign(mass, mass + n_);
     std::vector<double> rm(n_);
-    std::vector<double4> p(n_), v(n_);
     for(size_t i = 0; i < n_; ++i)
     {
         if(!(mass[i] > 0.0)) {throw std::invalid_argument("masses must be positive");}
         rm[i] = 1.0 / mass[i];
-        double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
-        if(box_.periodic)
-        {
-            // System::initialize wraps positions (System.hpp:63-67, BoundaryCondition.hpp:93-102)
-            if(x < box_.lower[0]) {x += box_.width[0];} else if(x >= box_.upper[0]) {x -= box_.width[0];}
-            if(y < box_.lower[1]) {y += box_.width[1];} else if(y >= box_.upper[1]) {y -= box_.width[1];}
-            if(z < box_.lower[2]) {z += box_.width[2];} else if(z >= box_.upper[2]) {z -= box_.width[2];}
-        }
-        p[i] = make_double4(x, y, z, 0.0);
-        v[i] = make_double4(vel[3 * i], vel[3 * i + 1], vel[3 * i + 2], 0.0);
     }
     upload(d_mass_, mass_.data(), n_);
     upload(d_rmass_, rm.data(), n_);
-    upload(d_pos_, p.data(), n_);
-    upload(d_vel_, v.data(), n_);
-    if(d_old_pos_) {upload(d_old_pos_, p.data(), n_);}   // g-BAOAB: the last step end is now
+    // System::initialize wraps positions (System.hpp:63-67, BoundaryCondition.hpp:93-102)
+    check(transfer_.upload(pos, d_pos_, n_, box_, stream_), "upload positions");
+    check(transfer_.upload(vel, d_vel_, n_, Box{}, stream_), "upload velocities");
+    if(d_old_pos_)   // g-BAOAB: the last step end is now
+    {
+        hipLaunchKernelGGL(k_copy_double4, dim3(blocks_for(n_, 256)), dim3(256), 0, stream_, (uint32_t)n_, d_pos_, d_old_pos_);
+    }
     hipLaunchKernelGGL(k_zero_double4, dim3(blocks_for(n_, 256)), dim3(256), 0, stream_, d_force_, (uint32_t)n_);
     check(hipGetLastError(), "set_state launch");
     sync();
@@ -202,7 +195,7 @@ void Engine::set_positions(const double* pos)
 {
     if(!pos) {throw std::invalid_argument("null position pointer");}
     if(!state_set_) {throw std::logic_error("set the state first");}
-    check(transfer_.upload_positions(pos, d_pos_, n_, box_, stream_), "upload positions");
+    check(transfer_.upload(pos, d_pos_, n_, box_, stream_), "upload positions");
 }
 
 void Engine::get_state(double* pos, double* vel, double* force)
@@ -359,7 +352,10 @@ void Engine::add_constraint(const char* topology, size_t n, const uint32_t* idx,
 // construct_molecules (Topology.hpp:280-317): only "bond" edges join molecules.
 void Engine::write_topology()
 {
-    adj_.assign(n_, {});
+    // no table of connections where nothing connects: 24 bytes a particle, kept with the engine
+    bool connected = con_.topo_kind >= 0;
+    for(const auto& L : locals_) {connected = connected || L.topo_kind >= 0;}
+    adj_.assign(connected ? n_ : 0, {});
     auto add = [&](uint32_t i, uint32_t j, int kind) {
         for(int s = 0; s < 2; ++s)
         {
@@ -408,6 +404,7 @@ void Engine::write_topology()
     uint32_t next = 0;
     for(size_t i = 0; i < n_; ++i)
     {
+        if(!connected) {mol_[i] = next++; continue;}
         for(const auto& e : adj_[i])
         {
             if(e.second != bond) {continue;}
@@ -433,6 +430,7 @@ void Engine::make_exclusions(GlobalIA& g)
         tmp.push_back((uint32_t)i);
         for(const auto& w : g.within)
         {
+            if(adj_.empty()) {break;}
             // depth-first walk over `kind` edges up to `dist` steps
             stack.clear();
             stack.emplace_back((uint32_t)i, w.second);
@@ -938,7 +936,7 @@ void Engine::initialize()
     // local tables: one segment per interaction
     std::vector<uint32_t> lidx;
     std::vector<double> lpar;
-    std::vector<std::vector<uint32_t>> per_particle(n_);
+    std::vector<std::vector<uint32_t>> per_particle(locals_.empty() ? 0 : n_);
     segtab_.n = 0;
     uint32_t block = 0, slot = 0, term = 0;
     for(size_t l = 0; l < locals_.size(); ++l)
@@ -1327,7 +1325,8 @@ void Engine::integrator_initialize()
     if(!has_T_) {throw std::out_of_range("Langevin integrator requires the `temperature` attribute");}
     const double kBT = kB_kcal() * T_;
     const double noise_coef = std::sqrt(2 * kB_kcal() * T_ / dt_);
-    std::vector<double> c1(n_), c2(n_), c3(n_);
+    const bool gjf = (integ_ == MJG_INTEG_GJF);   // the one integrator with a third coefficient
+    std::vector<double> c1(n_), c2(n_), c3(gjf ? n_ : 0);
     for(size_t i = 0; i < n_; ++i)
     {
         if(integ_ == MJG_INTEG_UNDERDAMPED)
@@ -1353,7 +1352,7 @@ void Engine::integrator_initialize()
     if(!d_c1_) {d_c1_ = dalloc<double>(n_); d_c2_ = dalloc<double>(n_); d_c3_ = dalloc<double>(n_);}
     upload(d_c1_, c1.data(), n_);
     upload(d_c2_, c2.data(), n_);
-    upload(d_c3_, c3.data(), n_);
+    upload(d_c3_, c3.data(), c3.size());
     if(integ_ == MJG_INTEG_GBAOAB) {setup_constraints();}
     forces(d_force_, false, -1, false);
     if(integ_ == MJG_INTEG_GBAOAB)

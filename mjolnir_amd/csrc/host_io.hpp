@@ -1,5 +1,5 @@
 // Transfers between the caller's arrays and the device state through pinned host memory: kernels
-// pack the wanted double4 arrays into x, y, z triples there (downloads) or take positions from
+// pack the wanted double4 arrays into x, y, z triples there (downloads) or take triples from
 // there (uploads), and the host copies between it and the caller's arrays.
 //
 // A transfer is bound by the host: one launch and one wait for a small system (three synchronous
@@ -32,16 +32,16 @@ k_pack_xyz(PackArgs a, uint32_t first, uint32_t n, double* __restrict__ out)
     }
 }
 
-// pos[first + i] = the triple in[3 i ..], wrapped into the box as System::initialize wraps it
-// (System.hpp:63-67, BoundaryCondition.hpp:93-102)
+// to[first + i] = the triple in[3 i ..], wrapped into the box as System::initialize wraps positions
+// (System.hpp:63-67, BoundaryCondition.hpp:93-102); a box that is not periodic leaves it as it is
 static __global__ void __launch_bounds__(256)
-k_unpack_positions(const double* __restrict__ in, uint32_t first, uint32_t n, Box box, double4* __restrict__ pos)
+k_unpack_xyz(const double* __restrict__ in, uint32_t first, uint32_t n, Box box, double4* __restrict__ to)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if(i >= n) {return;}
     double x = in[3 * (size_t)i], y = in[3 * (size_t)i + 1], z = in[3 * (size_t)i + 2];
     adjust_position(box, x, y, z);
-    pos[first + i] = make_double4(x, y, z, 0.0);
+    to[first + i] = make_double4(x, y, z, 0.0);
 }
 
 // Two pinned halves: while the host works on one, the device works on the other.  One owner (an
@@ -116,8 +116,8 @@ class StateTransfer
         return hipSuccess;
     }
 
-    // pos[i] = the caller's triple i, wrapped into the box; complete when it returns
-    hipError_t upload_positions(const double* from, double4* pos, size_t n, const Box& box, hipStream_t stream)
+    // to[i] = the caller's triple i, wrapped into the box; complete when it returns
+    hipError_t upload(const double* from, double4* to, size_t n, const Box& box, hipStream_t stream)
     {
         const size_t per = half_ / (3 * sizeof(double));
         const size_t chunks = (n + per - 1) / per;
@@ -131,8 +131,8 @@ class StateTransfer
             const size_t k = std::min(per, n - c * per);
             double* half = reinterpret_cast<double*>(static_cast<char*>(pin_) + (c & 1) * half_);
             std::memcpy(half, from + 3 * c * per, 3 * k * sizeof(double));
-            hipLaunchKernelGGL(k_unpack_positions, dim3((uint32_t)((k + 255) / 256)), dim3(256), 0, stream, half,
-                               (uint32_t)(c * per), (uint32_t)k, box, pos);
+            hipLaunchKernelGGL(k_unpack_xyz, dim3((uint32_t)((k + 255) / 256)), dim3(256), 0, stream, half,
+                               (uint32_t)(c * per), (uint32_t)k, box, to);
             hipError_t e = hipGetLastError();
             if(e == hipSuccess && chunks > 2) {e = hipEventRecord(ev_[c & 1], stream);}
             if(e != hipSuccess) {return e;}

@@ -353,3 +353,25 @@ def test_dilute_fluids_rebuild_with_enough_lanes(n, margin):
         best = min(best, (time.perf_counter() - t0) / 100)
     print(f"[gpu] dilute {n}, margin {margin}: {best * 1e6:.1f} us a step", flush=True)
     assert best < 60e-6
+
+
+@pytest.mark.parametrize("n", [1, 10922, 10923, 21845, 40000])
+def test_state_set_and_read_back_through_the_pinned_halves(n):
+    """Sizes around the particles of a half (10922 triples of positions): positions up to a box width outside come
+    back wrapped once, as the reference wraps them, velocities as they are, forces zero before the first call."""
+    import ctypes as C
+    from mjolnir_amd import capi
+    rng = np.random.default_rng(n)
+    lower, upper = np.array([-3.0, 0.0, 5.0]), np.array([9.0, 11.0, 18.0])
+    w = upper - lower
+    pos, vel = lower + w * rng.uniform(-0.9, 1.9, size=(n, 3)), rng.normal(size=(n, 3))
+    want = np.where(pos < lower, pos + w, np.where(pos >= upper, pos - w, pos))
+    L, h = capi.lib(), C.c_void_p()
+    assert L.mjg_engine_create(capi.FP64, capi.PERIODIC, lower, upper, n, 0, C.byref(h)) == capi.OK
+    try:
+        assert L.mjg_system_set_state(h, np.ones(n), pos, vel) == capi.OK
+        x, v, f = (np.full((n, 3), 7.0) for _ in range(3))
+        assert L.mjg_system_get_state(h, x.ctypes.data, v.ctypes.data, f.ctypes.data) == capi.OK
+    finally:
+        L.mjg_engine_destroy(h)
+    assert np.array_equal(x, want) and np.array_equal(v, vel) and not f.any()
