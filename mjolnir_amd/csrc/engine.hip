@@ -837,7 +837,7 @@ void Engine::launch_rebuilds(int force, uint32_t k)
                                g.d_cell_end, g.sb.keys, g.sb.vals, ctl);
             hipLaunchKernelGGL(k_cell_order, dim3(std::min(blocks_for(cells, 256 / kWave), kSortBlocks)), dim3(256), 0,
                                stream_, g.d_grid, g.d_cell_start, g.d_cell_end, g.sb.count, g.sb.vals, d_pos_,
-                               g.d_part, g.d_spart, g.d_spos, ctl);
+                               g.d_part, g.d_spart, g.d_spos, g.sb.ukeys, ctl);   // the unsorted keys are done with
         }
     }
     // the slot copies of the interactions that k_prep_small prepares (k_cell_order made the others')

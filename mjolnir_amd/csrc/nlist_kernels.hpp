@@ -267,13 +267,16 @@ __global__ void k_cell_place(const uint32_t* __restrict__ ukeys, uint32_t np, ui
 // participants of the cell before its own), then the particle and position of every slot (the slot
 // copies the list builds read), and the cell's count cleared.  One thread per cell sorting by
 // insertion in global memory took 410 us for the 19 participants of a cell of a liquid at
-// r_list = 15 A, half of a rebuild of 30,000 particles.  A cell of more than a wave's lanes is
-// still sorted that way.
+// r_list = 15 A, half of a rebuild of 30,000 particles.  A cell of more than a wave's lanes goes the
+// same way through `tmp`, kCrowd participants a lane at a time.  Participants crowd where an open
+// system's box is stretched by a few that flew off (an exploded chain): one lane's insertion took
+// 1.8 s a build for 5000 of them in one cell, and such a system rebuilds on every step.
+constexpr int kCrowd = 4;
 __global__ void __launch_bounds__(256)
 k_cell_order(const Grid* __restrict__ grid, const uint32_t* __restrict__ cell_start,
              const uint32_t* __restrict__ cell_end, uint32_t* __restrict__ count, uint32_t* __restrict__ svals,
              const double4* __restrict__ pos, const uint32_t* __restrict__ part, uint32_t* __restrict__ spart,
-             double4* __restrict__ spos, const ListCtl* __restrict__ ctl)
+             double4* __restrict__ spos, uint32_t* __restrict__ tmp, const ListCtl* __restrict__ ctl)
 {
     if(ctl->rebuild == 0) {return;}
     const uint32_t n = grid->ncell;
@@ -297,25 +300,35 @@ k_cell_order(const Grid* __restrict__ grid, const uint32_t* __restrict__ cell_st
             }
             continue;
         }
-        if(lane == 0)
+        for(uint32_t x0 = b; x0 < e; x0 += kCrowd * (uint32_t)kWave)
         {
-            for(uint32_t x = b + 1; x < e; ++x)
+            uint32_t v[kCrowd], at[kCrowd];
+#pragma unroll
+            for(int q = 0; q < kCrowd; ++q)
             {
-                const uint32_t v = svals[x];
-                uint32_t y = x;
-                while(y > b && svals[y - 1] > v)
-                {
-                    svals[y] = svals[y - 1];
-                    --y;
-                }
-                svals[y] = v;
+                const uint32_t x = x0 + q * (uint32_t)kWave + lane;
+                v[q] = (x < e) ? svals[x] : 0u;
+                at[q] = b;
             }
-            for(uint32_t x = b; x < e; ++x)
+            for(uint32_t y = b; y < e; ++y)
             {
-                const uint32_t i = part[svals[x]];
-                spart[x] = i;
-                spos[x] = pos[i];
+                const uint32_t o = svals[y];
+#pragma unroll
+                for(int q = 0; q < kCrowd; ++q) {at[q] += (o < v[q]) ? 1u : 0u;}
             }
+#pragma unroll
+            for(int q = 0; q < kCrowd; ++q)
+            {
+                if(x0 + q * (uint32_t)kWave + lane < e) {tmp[at[q]] = v[q];}
+            }
+        }
+        __threadfence_block();                               // the wave's lanes read what its others wrote
+        for(uint32_t x = b + lane; x < e; x += (uint32_t)kWave)
+        {
+            const uint32_t v = tmp[x], i = part[v];
+            svals[x] = v;
+            spart[x] = i;
+            spos[x] = pos[i];
         }
     }
 }
@@ -758,18 +771,26 @@ k_prep_small(const double4* __restrict__ pos, PrepSegTable tab, StepCtl* __restr
         sval[slot] = p;
     }
     __syncthreads();
+    // a participant's place is the number of participants of its cell before it
+    constexpr uint32_t kPer = kSmallMaxPart / 1024;
+    uint32_t val[kPer], at[kPer];
+#pragma unroll
+    for(uint32_t m = 0; m < kPer; ++m)
+    {
+        const uint32_t t = m * 1024 + tid;
+        if(t >= s.np) {continue;}
+        val[m] = sval[t];
+        const uint32_t c = key[val[m]], b = start[c], e = start[c + 1];
+        at[m] = b;
+        for(uint32_t y = b; y < e; ++y) {at[m] += (sval[y] < val[m]) ? 1u : 0u;}
+    }
+    __syncthreads();
+#pragma unroll
+    for(uint32_t m = 0; m < kPer; ++m) {if(m * 1024 + tid < s.np) {sval[at[m]] = val[m];}}
     for(uint32_t c = tid; c < ncell; c += nt)
     {
-        const uint32_t b = start[c], e = start[c + 1];
-        for(uint32_t a = b + 1; a < e; ++a)
-        {
-            const uint32_t v = sval[a];
-            uint32_t q = a;
-            while(q > b && sval[q - 1] > v) {sval[q] = sval[q - 1]; --q;}
-            sval[q] = v;
-        }
-        s.cell_start[c] = b;
-        s.cell_end[c] = e;
+        s.cell_start[c] = start[c];
+        s.cell_end[c] = start[c + 1];
     }
     __syncthreads();
     for(uint32_t t = tid; t < s.np; t += nt)

@@ -442,3 +442,30 @@ def test_steps_joined_and_separate_in_turn(n):
     d = x - xo
     d -= w * np.round(d / w)
     assert np.abs(d).max() < 1e-8 and np.abs(v - vo).max() < 1e-8 and np.abs(f - fo).max() < 1e-8 * np.abs(fo).max()
+
+
+@pytest.mark.parametrize("n", [70, 3000, 4096, 20000])
+def test_participants_crowded_into_one_cell(n):
+    """A particle far away from all others stretches an open system's cells until one holds the rest: up to 4096 the
+    one-workgroup rebuild, above it the counting sort.  The list is the all-pairs list; one lane's
+    sort took 1.8 s for 5000 of them and grows with the square."""
+    import time
+    from mjolnir_amd import capi
+    from mjolnir_amd.spec import GlobalSpec, IntegratorSpec, SystemSpec
+    rng = np.random.default_rng(n)
+    side = int(np.ceil((n - 1) ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n - 1] * 2.0
+    pos = np.concatenate([g, [[1e12, -1e12, 1e12]]])[rng.permutation(n)]
+    out = []
+    for partition in ("CellList", "VerletList"):
+        lj = GlobalSpec(potential="LennardJones", participants=np.arange(n), params=np.tile([1.0, 0.02], (n, 1)),
+                        cutoff=2.5, partition=partition, margin=0.1)
+        t0 = time.perf_counter()
+        e = capi.Engine(SystemSpec(boundary="unlimited", mass=np.ones(n), pos=pos, vel=np.zeros_like(pos),
+                                   attributes={"temperature": 1.0}, global_=[lj],
+                                   integrator=IntegratorSpec("BAOABLangevin", 0.01, np.full(n, 0.01), seed=3),
+                                   name=f"crowd_{n}"))
+        print(f"[gpu] {n} in one cell, {partition}: set up in {time.perf_counter() - t0:.3f} s", flush=True)
+        out.append((e.pairs(0), time.perf_counter() - t0))
+    assert len(out[0][0]) > n and np.array_equal(out[0][0], out[1][0])
+    assert out[0][1] < 3.0
