@@ -485,7 +485,8 @@ void Engine::alloc_list(GlobalIA& g, uint32_t cap)
 // grids.  In the mixed precision no axis of the box may be narrower than three list radii
 // (GlobalIA::one_image): the gather kernel serves those boxes.  Its staging capacity starts at twice the mean 27-cell neighbourhood and grows with the
 // largest one a build reports (ListCtl::maxnbr), up to what the LDS of one workgroup holds after
-// the kernel's static LDS (224 bytes in the current build; 4 KiB are set aside for it).
+// the kernel's static LDS (672 bytes in the stepping kernels, 224 for each of their three uses of the lists;
+// 4 KiB are set aside for it).
 constexpr uint32_t kTileMinNp = 16384;
 constexpr uint32_t kTileMaxCap = (uint32_t)((160 * 1024 - 4096) / kTileBytesPerParticle);
 static uint32_t tile_min_np()
@@ -498,7 +499,14 @@ static uint32_t tile_min_np()
 // blocks that leave at once take about 2 us longer than 256.
 constexpr uint32_t kSortBlocks = 256;
 
-// Largest interaction whose list k_forces keeps by brute force (np^2 / 2 distance tests a rebuild).
+// Largest interaction whose list k_forces keeps by brute force (np^2 distance tests a rebuild).  The line is
+// that of the one-workgroup rebuild, below the sizes where the one launch stops being the faster way: with
+// the line moved up, an FP64 step of a fluid took 12.3 us instead of the rebuild pipeline's 21.1 at 5000
+// particles, 14.0 instead of 21.7 at 8192, 19.1 instead of 23.5 at 12,000 and 24.0 instead of 26.2 at 16,000; at
+// m = 0.1, with five times the rebuilds, 16.4 instead of 22.9, 23.9 instead of 24.2, 36.0 instead of 24.8
+// and 59.1 instead of 26.8; a chain of 5000 beads 15.1 instead of 38.7, a duplex of 1500 bp 32.5 instead of
+// 73.6.  It has not been moved because a gather run above it is held bit for bit to the cell-tile run, whose
+// rows the pipeline orders by cell.
 constexpr size_t kSelfMaxPart = 4096;
 
 // lanes per participant: about six partners per lane, a power of two in [1, 64]

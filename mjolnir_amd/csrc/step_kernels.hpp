@@ -13,17 +13,21 @@
 // what counts is their number: two here, where separate kernels for the skin check, the cell sort,
 // the list build, the local terms, the pairs, each 3SPN2 interaction, the force sum and the
 // position update make 6 (a fluid) to 17 (a DNA duplex).  A rebuild by brute force is np^2 distance
-// tests without any ordering between blocks: 75 us at 4096 participants, where the cell sort and
-// the build from it took 180.  Measured per FP64 step, before and after: a fluid of 512 particles
-// 17.0 -> 9.4 us, of 4096 19.1 -> 11.4, a chain of 1000 beads 29.3 -> 12.5, a 200-bp duplex
-// 66 -> 28; mixed chain of 3001 beads 33 -> 14.5.
+// tests without any ordering between blocks: a launch with one takes 71 us at 4096 participants (6.9 without),
+// where the cell sort and the build from it took 180.  Measured per FP64 step, before and after: a fluid of 512
+// particles 17.0 -> 9.4 us, of 4096 18.9 -> 11.1, a chain of 1000 beads 27.5 -> 11.4, a 200-bp duplex
+// 64 -> 18; mixed chain of 3001 beads 29 -> 11.6.
 #pragma once
 #include "force_kernels.hpp"
 #include "nlist_kernels.hpp"
 
 namespace mjg
 {
-// the lists that k_forces keeps: their margins are settled by the next k_advance
+// the lists that k_forces keeps: their margins are settled by the next k_advance.  Four are what the largest
+// of the framework's own force fields has (3SPN2: excluded volume, Debye-Hueckel, base pairing, cross
+// stacking; four local interactions beside them); the table of them travels in the kernel's arguments.  A
+// system with more takes the separate launches (a chain of 1000 beads with five lists 29.7 us a step, with
+// its two 11.4).
 constexpr int kMaxSelfLists = 4;
 struct SelfLists
 {
@@ -230,7 +234,6 @@ k_backup(BackupArgs a)
 // all forces of a small system
 // ------------------------------------------------------------------------------------
 constexpr int kMaxSmallLocals = 8;
-constexpr int kSmallSeg = 8;         // blocks' runs: global interactions, local terms, noise
 
 // one global interaction: its rows and what keeps its list
 struct RowSeg
@@ -270,10 +273,10 @@ constexpr uint32_t kScanEx = 4096;    // exclusions staged by a block, shared ou
 // The rows of one block found among all participants, in participant order; the pairs are k_verlet's
 // (the same distance test, pair_allowed's rules).  A candidate near enough used to read the participant,
 // base and exclusion tables in a dependent chain of about 3 us, on nearly every round of a chain's or
-// a duplex's rows (251 us a rebuild of the 200-bp duplex); here a tile's tables are staged with its
-// positions, loaded while the tile before is tested, and a row keeps its own exclusions in LDS (an
-// exclusion holds both ways, so the owner's list decides).  Every thread of the block calls it;
-// `valid`: the thread's row exists.
+// a duplex's rows (251 us for a force launch of the 200-bp duplex with a rebuild, 92 now, 9.5 without one);
+// here a tile's tables are staged with its positions, loaded while the tile before is tested, and a row
+// keeps its own exclusions in LDS (an exclusion holds both ways, so the owner's list decides).  Every thread
+// of the block calls it; `valid`: the thread's row exists.
 __device__ __forceinline__ void self_build(const RowSeg& s, const Box& box, const double4* __restrict__ pos, uint32_t t,
                                            uint32_t l, bool valid)
 {
